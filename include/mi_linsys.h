@@ -214,8 +214,9 @@ int mi_spmv_dot_noalloc(mi_sys* sys, const double* x, double* y, double* d_dot, 
 int mi_spmv_shapes(int32_t* count, int32_t* dflt, int32_t* threads, int32_t* rows, int32_t* per, int32_t* vec);
 enum
 {
-    MI_SPMV_SHAPE_AUTO = -1, /* by the system's size (the default): the largest window whose count
-                                fills the GPU (1.5 windows per CU), else the full BSR             */
+    MI_SPMV_SHAPE_AUTO = -1, /* by the system's size (the default): windows small enough to fill the
+                                GPU with workgroups, from 64 rows above 16,384 block rows to 512
+                                rows; the full BSR up to 16,384 block rows                     */
     MI_SPMV_SHAPE_FULL = -2  /* the full BSR (both triangles, a row gather)                       */
 };
 /* The layout this system's SpMV uses: a window shape (an index of

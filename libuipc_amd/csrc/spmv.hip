@@ -664,7 +664,8 @@ struct WinShape
 #define MI_WIN_SHAPES(X)                                                                              \
     X(0, 512, 9, 2, 2) X(1, 256, 8, 3, 1) X(2, 512, 9, 2, 1) X(3, 256, 8, 2, 2) X(4, 256, 8, 2, 1) \
     X(5, 512, 9, 1, 1) X(6, 1024, 10, 1, 1) X(7, 256, 7, 2, 1) X(8, 256, 8, 4, 2) X(9, 512, 9, 4, 2) \
-    X(10, 1024, 9, 2, 2) X(11, 512, 9, 2, 4)  /* 11: FP32 systems' 512-row default */
+    X(10, 1024, 9, 2, 2) X(11, 512, 9, 2, 4)  /* 11: FP32 systems' 512-row default */ \
+    X(12, 512, 6, 1, 1) X(13, 256, 6, 2, 2) X(14, 256, 6, 1, 1) X(15, 256, 7, 2, 2) X(16, 256, 7, 2, 4)
 #define MI_WIN_ENTRY(i, nt, sh, per, vec) {nt, sh, per, vec},
 constexpr WinShape kWinShapes[] = {MI_WIN_SHAPES(MI_WIN_ENTRY)};
 #undef MI_WIN_ENTRY
@@ -816,21 +817,38 @@ int spmv_default_shape()
     return default_shape_index();
 }
 
-// the layout of a system of B block rows when none is set: the largest
-// window (512, 256 or 128 rows) whose count fills the chip, at least 1.5
-// windows per CU (one workgroup streams a window, so fewer windows leave
-// CUs idle: 8 windows of 512 rows ran a 4,096-row system on 8 CUs), else the
-// full BSR (spmv_shape_full)
+// The layout of a system of B block rows when none is set.  One workgroup
+// streams a window, so a small system needs small windows for workgroups to
+// fill the chip, and several workgroups per CU to even out its windows' block
+// counts; a large one needs large windows, which store fewer blocks twice.
+// us per product in a MAS part order (us of the layout this rule picked
+// before: 512-, 256- and 128-row windows at 1.5 windows per CU or more, else
+// the full BSR), grid^3 + contacts:
+//   FP64: 20^3 + 40k full 5.8; 33^3 + 150k 512 threads on 64 rows 15.8 (full
+//         21.5); 41^3 + 400k 256 on 64 rows 29.9 (35.6); 52^3 + 900k 256 on
+//         128 rows 56.5 (63.5); 61^3 + 1.2M 512 on 512 rows 78 (256 on 128: 79)
+//   FP32: 33^3 12.4 (15.3), 37^3 + 300k 16.9 (22.7); 41^3 one block per load
+//         21.6 (27.1), 46^3 + 500k 25.4 (27.6); 52^3 four blocks per load 37.6
+//         (46.8); 61^3 512 rows 55.6, 64^3 + 2M 64.1 (256 on 128: 59.5, 69.2)
+// In the caller's order (no MAS) the same choices measured 19.0 (21.8), 35.9
+// (40.9) and 71.2 (78.5) in FP64.  Up to 16,384 rows the full BSR's row
+// gather is as fast (20^3: 5.8 against 9.1) or near (25^3 + 90k: 12.0
+// against 10.1), and its sums do not depend on scheduling.
 int spmv_auto_shape(int64_t B, bool use32)
 {
     if(env_shape_index() >= 0)
         return env_shape_index();
-    const int64_t need   = (3 * (int64_t)device_cu_count() + 1) / 2;
-    // FP32 value planes: the 512-row shape with four blocks per 16-byte load
-    const int     cand[] = {use32 ? 11 : default_shape_index(), 3, 7};
-    for(int k : cand)
-        if((B + (int64_t(1) << kWinShapes[k].shift) - 1) >> kWinShapes[k].shift >= need)
-            return k;
+    struct Rule
+    {
+        int64_t rows;  // from this many block rows on
+        int     f64, f32;
+    };
+    // rows per CU (256 of them): 768, 448, 224 or 160, 64
+    static constexpr Rule rules[] = {{196608, 0, 11}, {114688, 15, 16}, {57344, 13, 14}, {40960, 13, 12}, {16385, 12, 12}};
+    const int64_t         rows    = B * 256 / std::max(1, device_cu_count());
+    for(const Rule& r : rules)
+        if(rows >= r.rows)
+            return use32 ? r.f32 : (r.f64 == 0 ? default_shape_index() : r.f64);
     return spmv_shape_full;
 }
 

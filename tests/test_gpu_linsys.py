@@ -252,6 +252,27 @@ def test_spmv_every_launch_shape(ctx, c1_contact, precision):
     ls.close()
 
 
+@pytest.mark.parametrize("precision", [abi.MI_FP64, abi.MI_FP32])
+@pytest.mark.parametrize("grid,rows", [(25, 0), (26, 64), (39, 64)])
+def test_spmv_layout_by_size(ctx, precision, grid, rows):
+    """the layout a system gets by its size (the full BSR up to 16,384 block
+    rows, 64-row windows above; the last window of 26^3 and 39^3 rows is a
+    partial one) and its product, against the oracle"""
+    s = synth.fem_system(grid, 2 * grid ** 2, seed=4)
+    ls = assembled(ctx, s, precision)
+    lay = ls.spmv_layout()
+    assert lay["window_rows"] == rows and lay["layout"] == ("window" if rows else "full")
+    orr, oc, ov, _ = O.convert_sym(s.block_rows, s.rows, s.cols, s.vals)
+    x = np.random.default_rng(9).standard_normal(s.n)
+    yref, dref = O.spmv_sym(s.block_rows, orr, oc, ov, x)
+    yd = ctx.alloc(s.n, np.float64)
+    d = ls.spmv_dot(ctx.to_device(x), yd)
+    tol = 1e-13 if precision == abi.MI_FP64 else 1e-6  # as test_spmv_dot
+    assert np.abs(yd.numpy() - yref).max() <= tol * np.abs(yref).max()
+    assert d == pytest.approx(dref, rel=tol * 10)
+    ls.close()
+
+
 def test_pcg_after_a_shape_change(ctx, c1_contact):
     """a solve captured in a HIP graph with one SpMV layout is not replayed
     after the layout changes (another window size, the full BSR, the size's
