@@ -11,8 +11,9 @@
 //   * the sort is a hand-written LSD radix sort (8-bit digits, wave64 ballot
 //     ranking, LDS-staged stable scatter) instead of CUB;
 //   * duplicates are summed sequentially in ascending source order by one
-//     thread per output block, so the values are deterministic (the reference
-//     sums in atomic arrival order, fast_segmental_reduce.h:23-26);
+//     thread per entry of the output block, so the values are deterministic
+//     (the reference sums in atomic arrival order,
+//     fast_segmental_reduce.h:23-26);
 //   * values land in 9 SoA planes (see BsrMatrix);
 //   * one host read-back (the unique count, to size the outputs) instead of two;
 //   * the upper BCOO is then transposed (the same radix sort on col * B + row
@@ -402,6 +403,9 @@ __global__ __launch_bounds__(kThreads) void rle_count_kernel(const int64_t* d_m,
         tile_cnt[blockIdx.x] = s;
 }
 
+constexpr int kSegTile = 256;  // sorted entries per tile of the segmented reduce
+constexpr int kSegTail = 96;   // entries past the tile staged with it
+
 template <typename KeyT>
 __global__ __launch_bounds__(kThreads) void rle_write_kernel(const int64_t*  d_m,
                                                             const KeyT*     keys,
@@ -409,7 +413,8 @@ __global__ __launch_bounds__(kThreads) void rle_write_kernel(const int64_t*  d_m
                                                             KeyCodec        kc,
                                                             int32_t*        out_rows,
                                                             int32_t*        out_cols,
-                                                            int32_t*        seg_start)
+                                                            int32_t*        seg_start,
+                                                            uint32_t*       seg_tile)
 {
     __shared__ KeyT     sk[kTile + 1];
     __shared__ int32_t  hp[kTile];
@@ -431,8 +436,12 @@ __global__ __launch_bounds__(kThreads) void rle_write_kernel(const int64_t*  d_m
             ++c;
         }
     }
-    uint32_t heads = 0;
-    uint32_t o     = block_exclusive_scan<kThreads>(c, lds, &heads);  // its barriers end every read of sk
+    uint32_t       heads = 0;
+    uint32_t       o     = block_exclusive_scan<kThreads>(c, lds, &heads);  // its barriers end every read of sk
+    const uint32_t g     = tile_off[blockIdx.x];
+    // the heads before every segment tile of the reduce
+    if(first % kSegTile == 0)
+        seg_tile[(base + first) / kSegTile] = g + o;
     // the heads' keys (in place, in order) and positions, then written out by
     // consecutive lanes
 #pragma unroll
@@ -444,7 +453,6 @@ __global__ __launch_bounds__(kThreads) void rle_write_kernel(const int64_t*  d_m
             ++o;
         }
     __syncthreads();
-    const uint32_t g = tile_off[blockIdx.x];
     for(uint32_t i = threadIdx.x; i < heads; i += kThreads)
     {
         int32_t r, c;
@@ -455,89 +463,169 @@ __global__ __launch_bounds__(kThreads) void rle_write_kernel(const int64_t*  d_m
     }
 }
 
-// one 72-byte FP64 triplet record (index src) by five 16-byte buffer loads
-// from the 16-byte boundary at or below it (odd records start 8 bytes past
-// one); the buffer's range check returns zeros past the array's end
-__device__ __forceinline__ void load_record64(__amdgpu_buffer_rsrc_t rs, int32_t src, double (&v)[9])
-{
-    typedef double d2v __attribute__((ext_vector_type(2)));
-    const uint32_t off = 72u * (uint32_t)src;
-    const uint32_t b   = off & ~15u;
-    const d2v      t0  = __builtin_bit_cast(d2v, __builtin_amdgcn_raw_buffer_load_b128(rs, b, 0, 0));
-    const d2v      t1  = __builtin_bit_cast(d2v, __builtin_amdgcn_raw_buffer_load_b128(rs, b + 16u, 0, 0));
-    const d2v      t2  = __builtin_bit_cast(d2v, __builtin_amdgcn_raw_buffer_load_b128(rs, b + 32u, 0, 0));
-    const d2v      t3  = __builtin_bit_cast(d2v, __builtin_amdgcn_raw_buffer_load_b128(rs, b + 48u, 0, 0));
-    const d2v      t4  = __builtin_bit_cast(d2v, __builtin_amdgcn_raw_buffer_load_b128(rs, b + 64u, 0, 0));
-    const bool     odd = (off & 8u) != 0;
-    v[0]               = odd ? t0.y : t0.x;
-    v[1]               = odd ? t1.x : t0.y;
-    v[2]               = odd ? t1.y : t1.x;
-    v[3]               = odd ? t2.x : t1.y;
-    v[4]               = odd ? t2.y : t2.x;
-    v[5]               = odd ? t3.x : t2.y;
-    v[6]               = odd ? t3.y : t3.x;
-    v[7]               = odd ? t4.x : t3.y;
-    v[8]               = odd ? t4.y : t4.x;
-}
-
-// ---- segmented reduce: one thread per unique block, duplicates summed in
-// FP64 in ascending source order (bit-identical to a sequential left fold of
-// the values as doubles).  The gathers of a group of 4 are issued before
-// their (ordered) additions.  TV: the triplet values' type;
-// kWide: FP64 records by 16-byte loads (T records, 72 T < 2^32).
-template <typename TV, bool kWide = false>
-__global__ __launch_bounds__(kThreads) void seg_reduce_kernel(int64_t        U,
+// ---- segmented reduce: duplicates summed in FP64 in ascending source order
+// (bit-identical to a sequential left fold of the values as doubles).  Bound
+// by the random gathers of whole records (72 or 36 bytes, m of them).
+//
+// A workgroup takes tiles of 256 sorted entries.  It owns the blocks whose
+// first entry lies in the tile and stages the tile's records, and those of the
+// next kSegTail entries (where its last block ends), in LDS: nine consecutive
+// lanes load one record, so a load instruction touches about as many cache lines
+// as it has records, and the records of one element that meet in a row of
+// the matrix come from the same lines at the same time.  One thread per
+// scalar of a block sums from LDS and writes consecutive
+// doubles.  The next tile's values are in flight (in registers) while a tile
+// is summed, and the sources and block starts of the one after it.
+// 32.8M triplets of the 64^3 + 2M contact system: 1.62 -> 0.78 ms (2.36 GB of
+// records; one thread per block gathering its records one by one before),
+// FP32 33^3 + 150k 91 -> 63 us, 11^3 + 3k 21 -> 8 us.  Tails of 64, 32 and 16
+// entries: 0.92, 1.21 and 1.45 ms (a diagonal block has about 50 entries and
+// runs past them), 128: 0.78; 4 or 8 workgroups per CU 0.78, 16 0.90.  Giving
+// each XCD consecutive tiles changed nothing.
+template <typename TV>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void seg_reduce_kernel(int64_t        U,
                                                              const int64_t* d_m,
-                                                             const int32_t* seg_start,
-                                                             const int32_t* srcs,
-                                                             const TV*      vals,
-                                                             double*        out,
-                                                             int64_t        T = 0)
+                                                             const int32_t* __restrict__ seg_start,
+                                                             const uint32_t* __restrict__ seg_tile,
+                                                             const int32_t* __restrict__ srcs,
+                                                             const TV* __restrict__ vals,
+                                                             double* out)
 {
-    const int64_t m = *d_m;
-    const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc((void*)vals, 0, kWide ? (int)(uint32_t)(72 * T) : 0, 0x00020000);
-    auto load = [&](int32_t src, double (&v)[9]) {
-        if constexpr(kWide)
-            load_record64(rs, src, v);
-        else
-        {
-            const TV* p = vals + 9 * (int64_t)src;
+    constexpr int kCap  = kSegTile + kSegTail;
+    constexpr int kLoad = (9 * kCap + kThreads - 1) / kThreads;
+    static_assert(kSegTile == kThreads && kSegTail <= kThreads, "one entry and one block start per thread");
+    __shared__ TV      sv[9 * kCap];
+    __shared__ int32_t ss[2][kCap];
+    __shared__ int32_t sb[2][kSegTile + 1];
+    const int32_t m   = (int32_t)*d_m;
+    const int32_t nt  = (m + kSegTile - 1) / kSegTile;
+    const int     tid = threadIdx.x;
+    auto tile_of = [&](int64_t k) -> int32_t {  // the workgroup's k-th tile (nt: none)
+        const int64_t t = k * gridDim.x + blockIdx.x;
+        return t < nt ? (int32_t)t : nt;
+    };
+    // indices of a tile: its entries' sources, its blocks' starts
+    int32_t  i_src = 0, i_tail = 0, i_sb = 0, i_end = 0;
+    uint32_t hu0 = 0, hu1 = 0;
+    auto heads = [&](int32_t t) {
+        hu0 = t < nt ? seg_tile[t] : 0;
+        hu1 = t < nt ? (t + 1 < nt ? seg_tile[t + 1] : (uint32_t)U) : 0;
+    };
+    auto index_load = [&](int32_t t) {  // uses hu0, hu1 of t
+        const int32_t e = t * kSegTile + tid;
+        i_src  = e < m ? srcs[e] : 0;
+        i_tail = tid < kSegTail && e + kSegTile < m ? srcs[e + kSegTile] : 0;
+        i_sb   = hu0 + tid < hu1 ? seg_start[hu0 + tid] : m;
+        i_end  = hu1 < U ? seg_start[hu1] : m;
+    };
+    auto index_store = [&](int s, int nb) {
+        ss[s][tid] = i_src;
+        if(tid < kSegTail)
+            ss[s][kSegTile + tid] = i_tail;
+        if(tid < nb)
+            sb[s][tid] = i_sb;
+        if(tid == 0)
+            sb[s][nb] = i_end;
+    };
+    TV v[kLoad];
+    auto vals_load = [&](int s, int32_t c0, int nb) {
+        const int f0 = nb ? 9 * (sb[s][0] - c0) : 0;
+        const int f1 = nb ? 9 * min(sb[s][nb] - c0, kCap) : 0;
 #pragma unroll
-            for(int q = 0; q < 9; ++q)
-                v[q] = (double)p[q];
+        for(int k = 0; k < kLoad; ++k)
+        {
+            const int f = k * kThreads + tid;
+            if(f >= f0 && f < f1)
+            {
+                const int r = f / 9;
+                v[k]        = vals[9 * (int64_t)ss[s][r] + (f - 9 * r)];
+            }
         }
     };
-    for(int64_t u = (int64_t)blockIdx.x * kThreads + threadIdx.x; u < U; u += (int64_t)gridDim.x * kThreads)
+    int32_t t0 = tile_of(0);
+    if(t0 >= nt)
+        return;
+    heads(t0);
+    uint32_t u0 = hu0;  // the current tile's blocks [u0, u0 + nb)
+    int      nb = (int)(hu1 - hu0);
+    index_load(t0);
+    index_store(0, nb);
+    int32_t t1 = tile_of(1);
+    heads(t1);
+    uint32_t n_u0 = hu0;
+    int      n_nb = (int)(hu1 - hu0);
+    index_load(t1);
+    __syncthreads();
+    vals_load(0, t0 * kSegTile, nb);
+    index_store(1, n_nb);
+    int32_t t2 = tile_of(2);
+    heads(t2);
+    __syncthreads();
+    for(int k = 0;; ++k)
     {
-        const int64_t b = seg_start[u];
-        const int64_t e = (u + 1 < U) ? (int64_t)seg_start[u + 1] : m;
-        double        acc[9];
-        load(srcs[b], acc);
-        int64_t k = b + 1;
-        for(; k + 4 <= e; k += 4)
+        const int     cur = k & 1;
+        const int32_t c0  = t0 * kSegTile;
+#pragma unroll
+        for(int q = 0; q < kLoad; ++q)
         {
-            double t[4][9];
-#pragma unroll
-            for(int g = 0; g < 4; ++g)
-                load(srcs[k + g], t[g]);
-#pragma unroll
-            for(int g = 0; g < 4; ++g)
-#pragma unroll
-                for(int q = 0; q < 9; ++q)
-                    acc[q] = acc[q] + t[g][q];
+            const int f = q * kThreads + tid;
+            if(f < 9 * kCap)
+                sv[f] = v[q];
         }
-        for(; k < e; ++k)
+        __syncthreads();
+        // the next tile's values, and the indices of the one after it
+        if(t1 < nt)
+            vals_load(cur ^ 1, t1 * kSegTile, n_nb);
+        const uint32_t nn_u0 = hu0;
+        const int      nn_nb = (int)(hu1 - hu0);
+        if(t2 < nt)
+            index_load(t2);
+        const int32_t t3 = tile_of(k + 3);
+        heads(t3);
+        for(int i = tid; i < 9 * nb; i += kThreads)
         {
-            double t[9];
-            load(srcs[k], t);
+            const int     j = i / 9, q = i - 9 * j;
+            int           e  = sb[cur][j] - c0;
+            const int     e1 = sb[cur][j + 1] - c0, el = min(e1, kCap);
+            double acc = (double)sv[9 * e++ + q];
+            for(; e + 4 <= el; e += 4)
+            {
+                const double w0 = (double)sv[9 * e + q], w1 = (double)sv[9 * e + 9 + q],
+                             w2 = (double)sv[9 * e + 18 + q], w3 = (double)sv[9 * e + 27 + q];
+                acc = acc + w0;
+                acc = acc + w1;
+                acc = acc + w2;
+                acc = acc + w3;
+            }
+            for(; e < el; ++e)
+                acc = acc + (double)sv[9 * e + q];
+            // a block running past the staged entries
+            for(; e + 8 <= e1; e += 8)
+            {
+                TV w[8];
 #pragma unroll
-            for(int q = 0; q < 9; ++q)
-                acc[q] = acc[q] + t[q];
+                for(int h = 0; h < 8; ++h)
+                    w[h] = vals[9 * (int64_t)srcs[c0 + e + h] + q];
+#pragma unroll
+                for(int h = 0; h < 8; ++h)
+                    acc = acc + (double)w[h];
+            }
+            for(; e < e1; ++e)
+                acc = acc + (double)vals[9 * (int64_t)srcs[c0 + e] + q];
+            out[upper_at(u0 + j, q)] = acc;
         }
-#pragma unroll
-        for(int q = 0; q < 9; ++q)
-            out[upper_at(u, q)] = acc[q];
+        if(t1 >= nt)
+            break;
+        __syncthreads();
+        if(t2 < nt)
+            index_store(cur, nn_nb);
+        t0   = t1;
+        t1   = t2;
+        t2   = t3;
+        u0   = n_u0;
+        nb   = n_nb;
+        n_u0 = nn_u0;
+        n_nb = nn_nb;
     }
 }
 
@@ -1197,25 +1285,30 @@ void MatrixConverter::convert(int32_t        B,
     out.cols.resize((size_t)(U > 0 ? U : 1), ratio);
     out.vals.resize((size_t)9 * out.rows.cap);
     seg_start_.resize((size_t)(U > 0 ? U : 1), ratio);
+    seg_tile_.resize((size_t)ntiles * (kTile / kSegTile), ratio);
     if(narrow)
         rle_write_kernel<uint32_t><<<ntiles, kThreads, 0, s>>>(d_m, key_ptr<uint32_t>(cur), tile_cnt_.data(),
                                                                codec(), out.rows.data(), out.cols.data(),
-                                                               seg_start_.data());
+                                                               seg_start_.data(), seg_tile_.data());
     else
         rle_write_kernel<uint64_t><<<ntiles, kThreads, 0, s>>>(d_m, key_ptr<uint64_t>(cur), tile_cnt_.data(),
                                                                codec(), out.rows.data(), out.cols.data(),
-                                                               seg_start_.data());
+                                                               seg_start_.data(), seg_tile_.data());
 
     // 7-8. segmented reduce over the sorted permutation (1652-1698)
-    if(U > 0 && vals32)
-        seg_reduce_kernel<float><<<grid_of(U), kThreads, 0, s>>>(
-            U, d_m, seg_start_.data(), srcs_[cur].data(), static_cast<const float*>(vals), out.vals.data());
-    else if(U > 0 && 72 * T + 16 < ((int64_t)1 << 32))
-        seg_reduce_kernel<double, true><<<grid_of(U), kThreads, 0, s>>>(
-            U, d_m, seg_start_.data(), srcs_[cur].data(), static_cast<const double*>(vals), out.vals.data(), T);
-    else if(U > 0)
-        seg_reduce_kernel<double><<<grid_of(U), kThreads, 0, s>>>(
-            U, d_m, seg_start_.data(), srcs_[cur].data(), static_cast<const double*>(vals), out.vals.data());
+    if(U > 0)
+    {
+        // as many workgroups as are resident at once (4 per CU)
+        const int  nseg   = std::min(ceil_div(T, kSegTile), device_cu_count() * 4);
+        const auto reduce = [&](auto* v) {
+            seg_reduce_kernel<<<nseg, kThreads, 0, s>>>(U, d_m, seg_start_.data(), seg_tile_.data(),
+                                                        srcs_[cur].data(), v, out.vals.data());
+        };
+        if(vals32)
+            reduce(static_cast<const float*>(vals));
+        else
+            reduce(static_cast<const double*>(vals));
+    }
     row_ptr_kernel<<<grid_of(U + 1), kThreads, 0, s>>>(nullptr, U, out.rows.data(), out.row_ptr.data(), B);
 
     // the transpose of the off-diagonal upper blocks (the lower triangle)

@@ -125,6 +125,28 @@ def test_convert_random_bitexact(ctx, B, T, seed):
     check_bcoo_bitexact(assembled(ctx, s), s)
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("runs", [[1], [256], [255, 2, 300], [352, 1, 353, 96, 97, 1], [3000, 5, 1, 12000], [1] * 1500])
+def test_convert_runs_of_duplicates(ctx, dtype, runs):
+    """runs of equal keys around the sizes the segmented reduce stages (tiles
+    of 256 sorted entries and 96 past them): the sums are the sequential fold
+    in source order, bit for bit"""
+    rng = np.random.default_rng(len(runs) + sum(runs))
+    B = len(runs) + 1
+    at = np.repeat(np.arange(len(runs), dtype=np.int32), runs)
+    order = rng.permutation(at.size)
+    rows = at[order]
+    cols = (rows + (rows % 2)).astype(np.int32)  # diagonal and off-diagonal blocks
+    vals = (rng.standard_normal((at.size, 9)) * 10.0 ** rng.integers(-6, 6, (at.size, 1))).astype(dtype)
+    ls = LinearSystem(ctx, B, abi.MI_FP32 if dtype == np.float32 else abi.MI_FP64)
+    ls.assemble(ctx.to_device(rows), ctx.to_device(cols), ctx.to_device(vals))
+    r, c, v, rp = ls.export_bcoo()
+    orr, oc, ov, orp = O.convert_sym(B, rows, cols, vals.astype(np.float64))
+    assert np.array_equal(r, orr) and np.array_equal(c, oc) and np.array_equal(rp, orp)
+    assert np.array_equal(v.view(np.uint64), ov.reshape(v.shape).view(np.uint64))
+    ls.close()
+
+
 def test_convert_empty_and_reassemble(ctx, c1):
     ls = LinearSystem(ctx, 10)
     z = ctx.alloc(1, np.int32)
