@@ -25,10 +25,11 @@ namespace mi
 {
 namespace
 {
-constexpr int kThreads = 256;
-constexpr int kItems   = 16;
-constexpr int kTile    = kThreads * kItems;  // 4096 keys per tile
-constexpr int kWaves   = kThreads / kWave;
+constexpr int kThreads   = 256;
+constexpr int kItems     = 16;
+constexpr int kTileItems = kItems;
+constexpr int kTile      = kThreads * kItems;  // 4096 keys per tile
+constexpr int kWaves     = kThreads / kWave;
 
 // kept entries and their sort keys.  Mode 0: the triplet filter of
 // matrix_converter.inl:142 (plus a bound on col, which the reference leaves
@@ -101,23 +102,61 @@ __global__ __launch_bounds__(kThreads) void cv_count_kernel(int64_t        T,
     }
 }
 
-// ---- single-workgroup exclusive scan (n up to a few 100k), total -> *total
+// Exclusive scan of n consecutive values by one workgroup of NT threads, in
+// place, rounds of 16 NT values: consecutive lanes move consecutive values
+// between memory and LDS, a thread sums 16 consecutive ones (padded by one
+// word in 16, so that they lie in different banks).  Returns the total.
+constexpr int kScanItems = 16;
+template <int NT>
+__device__ __forceinline__ uint32_t scan_span(uint32_t* data, int64_t n, uint32_t* sv, uint32_t* lds)
+{
+    uint32_t carry = 0;
+    for(int64_t base = 0; base < n; base += NT * kScanItems)
+    {
+#pragma unroll
+        for(int k = 0; k < kScanItems; ++k)
+        {
+            const int t       = k * NT + (int)threadIdx.x;
+            sv[t + (t >> 4)] = base + t < n ? data[base + t] : 0u;
+        }
+        __syncthreads();
+        const int first = (int)threadIdx.x * (kScanItems + 1);
+        uint32_t  sum   = 0;
+#pragma unroll
+        for(int k = 0; k < kScanItems; ++k)
+            sum += sv[first + k];
+        uint32_t tot;
+        uint32_t e = carry + block_exclusive_scan<NT>(sum, lds, &tot);
+#pragma unroll
+        for(int k = 0; k < kScanItems; ++k)
+        {
+            const uint32_t v = sv[first + k];
+            sv[first + k]    = e;
+            e += v;
+        }
+        carry += tot;
+        __syncthreads();
+#pragma unroll
+        for(int k = 0; k < kScanItems; ++k)
+        {
+            const int t = k * NT + (int)threadIdx.x;
+            if(base + t < n)
+                data[base + t] = sv[t + (t >> 4)];
+        }
+        __syncthreads();
+    }
+    return carry;
+}
+
+// ---- single-workgroup exclusive scan (n up to 64k), total -> *total (one
+// value per thread and round took 24 us for 36k values)
 __global__ __launch_bounds__(1024) void scan_small_kernel(uint32_t* data, int64_t n, int64_t* total)
 {
+    __shared__ uint32_t sv[1024 * (kScanItems + 1)];
     __shared__ uint32_t lds[1024 / kWave + 1];
-    uint32_t            carry = 0;
-    for(int64_t base = 0; base < n; base += 1024)
-    {
-        int64_t  i = base + threadIdx.x;
-        uint32_t v = i < n ? data[i] : 0u;
-        uint32_t tot;
-        uint32_t e = block_exclusive_scan<1024>(v, lds, &tot);
-        if(i < n)
-            data[i] = carry + e;
-        carry += tot;
-    }
+    const uint32_t      tot = scan_span<1024>(data, n, sv, lds);
     if(threadIdx.x == 0 && total)
-        *total = (int64_t)carry;
+        *total = (int64_t)tot;
 }
 
 // ---- large exclusive scan: per-chunk sums, scan of sums, down-sweep
@@ -230,14 +269,30 @@ struct TripletSource
     }
 };
 
-// ---- radix sort: tile histogram (digit-major layout hist[d * ntiles + tile])
-template <typename KeyT, typename Src>
+// ---- radix sort: the digit counts of every tile and where each tile's runs
+// start.  Many tiles: hist[d * ntiles + tile], each digit's row scanned over
+// the tiles by a workgroup of its own (rs_rows_kernel), the digits' totals
+// scanned by every scatter workgroup: three launches per pass (a general scan
+// of the 256 ntiles counts took three by itself, or one of up to 24 us).  Up to
+// kFewKeys keys, where a pass is little more than its launches and its tiles'
+// serial rounds, tiles of 1,024 keys and hist[tile * 256 + d], which every
+// scatter workgroup sums over the tiles by itself: two launches.
+// (Counting the next pass's digits in the scatter, by global atomics at the
+// keys' new places, was slower: 81k keys' assembly 239 -> 368 us, the keys of
+// a run meet in a few counters.)
+constexpr int     kFewItems = 4;
+constexpr int     kFewTile  = kThreads * kFewItems;
+constexpr int64_t kFewKeys  = 128 * kFewTile;
+
+template <typename KeyT, typename Src, bool kFew>
 __global__ __launch_bounds__(kThreads) void rs_hist_kernel(Src           src,
                                                           int           shift,
                                                           uint32_t      dmask,
                                                           uint32_t*     hist,
                                                           int           ntiles)
 {
+    constexpr int kItems = kFew ? kFewItems : kTileItems;
+    constexpr int kTile  = kThreads * kItems;
     __shared__ uint32_t h[256];
     h[threadIdx.x] = 0;
     __syncthreads();
@@ -252,7 +307,21 @@ __global__ __launch_bounds__(kThreads) void rs_hist_kernel(Src           src,
             atomicAdd(&h[(uint32_t)(key >> shift) & dmask], 1u);
     }
     __syncthreads();
-    hist[(int64_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+    if constexpr(kFew)
+        hist[(int64_t)blockIdx.x * 256 + threadIdx.x] = h[threadIdx.x];
+    else
+        hist[(int64_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+}
+
+// exclusive scan of digit blockIdx.x's counts over the tiles, in place; its
+// total -> totals[digit]
+__global__ __launch_bounds__(kThreads) void rs_rows_kernel(uint32_t* hist, int ntiles, uint32_t* totals)
+{
+    __shared__ uint32_t sv[kThreads * (kScanItems + 1)];
+    __shared__ uint32_t lds[kWaves + 1];
+    const uint32_t      tot = scan_span<kThreads>(hist + (int64_t)blockIdx.x * ntiles, ntiles, sv, lds);
+    if(threadIdx.x == 0)
+        totals[blockIdx.x] = tot;
 }
 
 __device__ __forceinline__ uint64_t lanemask_lt64()
@@ -264,15 +333,19 @@ __device__ __forceinline__ uint64_t lanemask_lt64()
 // of its contiguous quarter of the tile in order (ballot-matched peers +
 // per-wave digit counters), the tile is reordered by digit in LDS, then each
 // digit run is written out contiguously.
-template <typename KeyT, typename Src>
+// totals: the digits' totals (many tiles).
+template <typename KeyT, typename Src, bool kFew>
 __global__ __launch_bounds__(kThreads) void rs_scatter_kernel(Src             src,
                                                              KeyT*           kout,
                                                              int32_t*        vout,
                                                              int             shift,
                                                              uint32_t        dmask,
-                                                             const uint32_t* hist_scan,
-                                                             int             ntiles)
+                                                             const uint32_t* __restrict__ hist,
+                                                             int             ntiles,
+                                                             const uint32_t* __restrict__ totals)
 {
+    constexpr int       kItems = kFew ? kFewItems : kTileItems;
+    constexpr int       kTile  = kThreads * kItems;
     __shared__ KeyT     sk[kTile];
     __shared__ int32_t  sv[kTile];
     __shared__ uint32_t wcnt[kWaves][256];
@@ -289,6 +362,23 @@ __global__ __launch_bounds__(kThreads) void rs_scatter_kernel(Src             sr
 #pragma unroll
     for(int q = 0; q < kWaves; ++q)
         wcnt[q][threadIdx.x] = 0;
+    // this digit's count in all tiles and in the tiles before this one
+    uint32_t dtotal = 0, dbefore = 0;
+    if constexpr(kFew)
+    {
+#pragma unroll 16
+        for(int t = 0; t < ntiles; ++t)
+        {
+            const uint32_t c = hist[t * 256 + (int)threadIdx.x];
+            dtotal += c;
+            dbefore += t < (int)blockIdx.x ? c : 0u;
+        }
+    }
+    else
+    {
+        dtotal  = totals[threadIdx.x];
+        dbefore = hist[(int64_t)threadIdx.x * ntiles + blockIdx.x];
+    }
     __syncthreads();
 
     KeyT           key[kItems];
@@ -339,7 +429,7 @@ __global__ __launch_bounds__(kThreads) void rs_scatter_kernel(Src             sr
         }
         uint32_t e = block_exclusive_scan<kThreads>(acc, lds, &tile_total);
         dstart[d]  = e;
-        gbase[d]   = hist_scan[(int64_t)d * ntiles + blockIdx.x];
+        gbase[d]   = block_exclusive_scan<kThreads>(dtotal, lds, (uint32_t*)nullptr) + dbefore;
     }
     __syncthreads();
 #pragma unroll
@@ -630,9 +720,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 }
 
 // ---- BSR row offsets from sorted rows: row_ptr[r] = first u with rows[u] >= r
-__global__ __launch_bounds__(kThreads) void row_ptr_kernel(const int64_t* d_n, int64_t nmax, const int32_t* rows, int32_t* row_ptr, int32_t B)
+__global__ __launch_bounds__(kThreads) void row_ptr_kernel(int64_t U, const int32_t* rows, int32_t* row_ptr, int32_t B)
 {
-    const int64_t U = d_n ? *d_n : nmax;
     for(int64_t u = (int64_t)blockIdx.x * kThreads + threadIdx.x; u <= U; u += (int64_t)gridDim.x * kThreads)
     {
         int32_t prev = (u == 0) ? -1 : rows[u - 1];
@@ -642,19 +731,26 @@ __global__ __launch_bounds__(kThreads) void row_ptr_kernel(const int64_t* d_n, i
     }
 }
 
-// ---- full BSR: lower part (transposed upper blocks, sorted by (col, row)) then
-// upper part of each row
+// the same for the lower entries, from their sorted keys
 template <typename KeyT>
-__global__ void unpack_lower_kernel(const int64_t* d_n, const KeyT* keys, KeyCodec kc, int32_t* lrow)
+__global__ __launch_bounds__(kThreads) void lower_ptr_kernel(const int64_t* d_n, const KeyT* __restrict__ keys,
+                                                            KeyCodec kc, int32_t* lower_ptr, int32_t B)
 {
     const int64_t n = *d_n;
-    for(int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x)
+    for(int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x; k <= n; k += (int64_t)gridDim.x * kThreads)
     {
-        int32_t lr, lc;
-        kc.lo_rc((uint64_t)keys[k], lr, lc);
-        lrow[k] = lr;
+        int32_t prev = -1, cur = B, lc;
+        if(k > 0)
+            kc.lo_rc((uint64_t)keys[k - 1], prev, lc);
+        if(k < n)
+            kc.lo_rc((uint64_t)keys[k], cur, lc);
+        for(int32_t r = prev + 1; r <= cur; ++r)
+            lower_ptr[r] = (int32_t)k;
     }
 }
+
+// ---- full BSR: lower part (transposed upper blocks, sorted by (col, row)) then
+// upper part of each row
 
 // chunk_row[c] = the first row whose first full-BSR block is at or after
 // c kChunkStep (binary search in full_ptr); chunk_row[nchunks] = B
@@ -997,9 +1093,9 @@ int radix_sort_from(First           first,
                     int32_t*        v1,
                     const int64_t*  d_n,
                     int64_t         nmax,
+                    int             low,
                     int             bits,
                     DBuf<uint32_t>& hist,
-                    DBuf<uint32_t>& chunk,
                     hipStream_t     s);
 
 // compaction + stable radix sort of (key, source) pairs; returns the buffer
@@ -1019,7 +1115,7 @@ int MatrixConverter::compact_sort(int64_t        n,
     keys_[1].resize((size_t)n, ratio);
     srcs_[0].resize((size_t)n, ratio);
     srcs_[1].resize((size_t)n, ratio);
-    hist_.resize((size_t)256 * ntiles, ratio);
+    hist_.resize((size_t)256 * (std::max(ntiles, (int)(kFewKeys / kFewTile)) + 1), ratio);
     if(!(MODE == 0 && counted_))
         cv_count_kernel<MODE><<<ntiles, kThreads, 0, s>>>(n, rows, cols, B, tile_cnt_.data(), nullptr);
     counted_ = false;
@@ -1029,9 +1125,12 @@ int MatrixConverter::compact_sort(int64_t        n,
     // compaction (the kept count, *d_count, from the tile counts) and a stable
     // LSD radix sort (matrix_converter.inl:1579-1616) on the key's bits, whose
     // first pass reads the triplets' (row, col) and skips the dropped entries
+    // (mode 1: the upper blocks come in row order, so a stable sort by column
+    // alone gives (column, row))
     TripletSource<MODE, KeyT> first{rows, cols, n, B, codec_};
-    return radix_sort_from<KeyT>(first, k0, srcs_[0].data(), k1, srcs_[1].data(), d_count, n, key_bits_, hist_,
-                                 chunk_, s);
+    const int                 low  = MODE == 1 ? codec_.lo_shift() : 0;
+    const int                 bits = MODE == 1 ? low + key_bits_for((uint64_t)std::max(B - 1, 1)) : key_bits_;
+    return radix_sort_from<KeyT>(first, k0, srcs_[0].data(), k1, srcs_[1].data(), d_count, n, low, bits, hist_, s);
 }
 
 void MatrixConverter::build_window(BsrMatrix& A, int shape, bool want32, double ratio, hipStream_t s)
@@ -1118,7 +1217,7 @@ void MatrixConverter::build_window(BsrMatrix& A, int shape, bool want32, double 
     A.has_win = true;
 }
 
-// stable LSD passes of 8 bits; the first reads `first` (pairs or triplets),
+// stable LSD passes of 8 bits over the key bits [low, bits); the first reads `first` (pairs or triplets),
 // the rest ping-pong between the buffers; returns the buffer holding the result
 template <typename KeyT, typename First>
 int radix_sort_from(First           first,
@@ -1128,30 +1227,39 @@ int radix_sort_from(First           first,
                     int32_t*        v1,
                     const int64_t*  d_n,
                     int64_t         nmax,
+                    int             low,
                     int             bits,
                     DBuf<uint32_t>& hist,
-                    DBuf<uint32_t>& chunk,
                     hipStream_t     s)
 {
-    const int ntiles = ceil_div(nmax, kTile);
+    const bool few    = nmax <= kFewKeys;
+    const int  ntiles = ceil_div(nmax, few ? kFewTile : kTile);
     if(ntiles == 0)
         return 0;
-    hist.resize((size_t)256 * ntiles);
-    KeyT*    kb[2] = {k0, k1};
-    int32_t* vb[2] = {v0, v1};
-    int      cur   = 0;
-    for(int shift = 0; shift < bits; shift += 8)
+    hist.resize((size_t)256 * (ntiles + 1));  // the counts, the digits' totals
+    uint32_t* totals = hist.data() + (size_t)256 * ntiles;
+    KeyT*     kb[2]  = {k0, k1};
+    int32_t*  vb[2]  = {v0, v1};
+    int       cur    = 0;
+    for(int shift = low; shift < bits; shift += 8)
     {
-        int      w     = (bits - shift) < 8 ? (bits - shift) : 8;
-        uint32_t dmask = (1u << w) - 1u;
-        auto     pass  = [&](auto src) {
+        const uint32_t dmask = (1u << std::min(8, bits - shift)) - 1u;
+        auto           pass  = [&](auto src) {
             using Src = decltype(src);
-            rs_hist_kernel<KeyT, Src><<<ntiles, kThreads, 0, s>>>(src, shift, dmask, hist.data(), ntiles);
-            scan_exclusive(hist.data(), (int64_t)256 * ntiles, chunk, nullptr, s);
-            rs_scatter_kernel<KeyT, Src><<<ntiles, kThreads, 0, s>>>(src, kb[cur ^ 1], vb[cur ^ 1], shift, dmask,
-                                                                     hist.data(), ntiles);
+            auto go   = [&](auto tag) {
+                constexpr bool kFew = decltype(tag)::value;
+                rs_hist_kernel<KeyT, Src, kFew><<<ntiles, kThreads, 0, s>>>(src, shift, dmask, hist.data(), ntiles);
+                if(!kFew)
+                    rs_rows_kernel<<<256, kThreads, 0, s>>>(hist.data(), ntiles, totals);
+                rs_scatter_kernel<KeyT, Src, kFew><<<ntiles, kThreads, 0, s>>>(src, kb[cur ^ 1], vb[cur ^ 1], shift,
+                                                                               dmask, hist.data(), ntiles, totals);
+            };
+            if(few)
+                go(std::true_type{});
+            else
+                go(std::false_type{});
         };
-        if(shift == 0)
+        if(shift == low)
             pass(first);
         else
             pass(PairSource<KeyT>{d_n, kb[cur], vb[cur]});
@@ -1169,10 +1277,9 @@ int radix_sort_pairs_t(KeyT*           k0,
                        int64_t         nmax,
                        int             bits,
                        DBuf<uint32_t>& hist,
-                       DBuf<uint32_t>& chunk,
                        hipStream_t     s)
 {
-    return radix_sort_from<KeyT>(PairSource<KeyT>{d_n, k0, v0}, k0, v0, k1, v1, d_n, nmax, bits, hist, chunk, s);
+    return radix_sort_from<KeyT>(PairSource<KeyT>{d_n, k0, v0}, k0, v0, k1, v1, d_n, nmax, 0, bits, hist, s);
 }
 
 int radix_sort_pairs(uint64_t*       k0,
@@ -1183,10 +1290,9 @@ int radix_sort_pairs(uint64_t*       k0,
                      int64_t         nmax,
                      int             bits,
                      DBuf<uint32_t>& hist,
-                     DBuf<uint32_t>& chunk,
                      hipStream_t     s)
 {
-    return radix_sort_pairs_t<uint64_t>(k0, v0, k1, v1, d_n, nmax, bits, hist, chunk, s);
+    return radix_sort_pairs_t<uint64_t>(k0, v0, k1, v1, d_n, nmax, bits, hist, s);
 }
 
 void exclusive_scan_u32(uint32_t* data, int64_t n, DBuf<uint32_t>& chunk, int64_t* d_total, hipStream_t s)
@@ -1309,21 +1415,19 @@ void MatrixConverter::convert(int32_t        B,
         else
             reduce(static_cast<const double*>(vals));
     }
-    row_ptr_kernel<<<grid_of(U + 1), kThreads, 0, s>>>(nullptr, U, out.rows.data(), out.row_ptr.data(), B);
+    row_ptr_kernel<<<grid_of(U + 1), kThreads, 0, s>>>(U, out.rows.data(), out.row_ptr.data(), B);
 
     // the transpose of the off-diagonal upper blocks (the lower triangle)
     const int tcur = narrow ? compact_sort<1, uint32_t>(U, out.rows.data(), out.cols.data(), B, d_off, ratio, s)
                             : compact_sort<1, uint64_t>(U, out.rows.data(), out.cols.data(), B, d_off, ratio, s);
     tcur_          = tcur;
-    lower_rows_.resize((size_t)(U > 0 ? U : 1), ratio);
     lower_ptr_.resize((size_t)B + 1, ratio);
     if(narrow)
-        unpack_lower_kernel<uint32_t><<<grid_of(U), kThreads, 0, s>>>(d_off, key_ptr<uint32_t>(tcur), codec(),
-                                                                      lower_rows_.data());
+        lower_ptr_kernel<uint32_t><<<grid_of(U + 1), kThreads, 0, s>>>(d_off, key_ptr<uint32_t>(tcur), codec(),
+                                                                       lower_ptr_.data(), B);
     else
-        unpack_lower_kernel<uint64_t><<<grid_of(U), kThreads, 0, s>>>(d_off, key_ptr<uint64_t>(tcur), codec(),
-                                                                      lower_rows_.data());
-    row_ptr_kernel<<<grid_of(U + 1), kThreads, 0, s>>>(d_off, U, lower_rows_.data(), lower_ptr_.data(), B);
+        lower_ptr_kernel<uint64_t><<<grid_of(U + 1), kThreads, 0, s>>>(d_off, key_ptr<uint64_t>(tcur), codec(),
+                                                                       lower_ptr_.data(), B);
     out.has_win  = false;
     out.has_full = false;
     if(build_full)

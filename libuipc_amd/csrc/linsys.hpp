@@ -80,7 +80,7 @@ constexpr int kWinShiftMax = 15;  // window offsets are 15-bit fields of the inn
 // diagonal and the rows and offsets fit in 32 bits, (row << bb) | (col - row)
 // on 32 bits -- the same order, sorted in fewer passes of two thirds the
 // bytes.  The transposed (lower) entries of the off-diagonal upper blocks sort
-// by (col, row): col * B + row, or (col << bb) | (row - col + band).
+// by (col, row): (col << 32) | row, or (col << bb) | (row - col + band).
 struct KeyCodec
 {
     uint64_t B    = 0;
@@ -92,8 +92,10 @@ struct KeyCodec
     }
     __host__ __device__ __forceinline__ uint64_t lo(int32_t r, int32_t c) const
     {
-        return bb ? ((uint64_t)c << bb) | (uint64_t)(r - c + band) : (uint64_t)c * B + (uint64_t)r;
+        return bb ? ((uint64_t)c << bb) | (uint64_t)(r - c + band) : ((uint64_t)c << 32) | (uint64_t)r;
     }
+    // the lower key's bits from here on are the column of the upper block
+    int lo_shift() const { return bb ? bb : 32; }
     __host__ __device__ __forceinline__ void up_rc(uint64_t k, int32_t& r, int32_t& c) const
     {
         if(bb)
@@ -117,8 +119,8 @@ struct KeyCodec
         }
         else
         {
-            lr = (int32_t)(k / B);
-            lc = (int32_t)(k - (uint64_t)lr * B);
+            lr = (int32_t)(k >> 32);
+            lc = (int32_t)(k & 0xffffffffu);
         }
     }
 };
@@ -189,7 +191,7 @@ class MatrixConverter
     DBuf<uint32_t> hist_, chunk_;
     DBuf<uint32_t> tile_cnt_;
     DBuf<uint32_t> seg_tile_;  // unique blocks before every tile of the segmented reduce
-    DBuf<int32_t>  seg_start_, lower_rows_, lower_ptr_;
+    DBuf<int32_t>  seg_start_, lower_ptr_;
     DBuf<int64_t>  counts_;  // [0] kept triplets, [1] U, [2] off-diagonal upper blocks, [3] full, [4] window blocks
     int            tcur_ = 0;  // buffer of the transposed (lower) sort
     KeyCodec       codec_{};
@@ -215,7 +217,6 @@ int radix_sort_pairs(uint64_t*       k0,
                      int64_t         nmax,
                      int             bits,
                      DBuf<uint32_t>& hist,
-                     DBuf<uint32_t>& chunk,
                      hipStream_t     s);
 // bits needed for keys up to max_key
 int radix_key_bits(uint64_t max_key);

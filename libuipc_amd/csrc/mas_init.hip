@@ -515,7 +515,7 @@ void build_adjacency_device(int32_t          V,
         MI_HIP(hipMemcpyAsync(cnt.data(), &E, sizeof(int64_t), hipMemcpyHostToDevice, s));
         const int bits = radix_key_bits((uint64_t)V * (uint64_t)V);
         const int cur  = radix_sort_pairs(keys[0].data(), vals[0].data(), keys[1].data(), vals[1].data(), cnt.data(),
-                                          E, bits, hist, chunk, s);
+                                          E, bits, hist, s);
         adj_head_kernel<<<grid_n(E), kT, 0, s>>>(keys[cur].data(), E, V, head.data(), out.nnum.data());
         exclusive_scan_u32(head.data(), E, chunk, cnt.data() + 1, s);
         out.M = read_back(cnt.data() + 1, s);

@@ -348,7 +348,7 @@ int32_t mesh_partition_device(int32_t        V,
         cpair_kernel<<<grid_p(V), kT, 0, s>>>(V, adj.nstart.data(), adj.nnum.data(), adj.nlist.data(), cv.data(),
                                               keys[0].data());
         const int cur = radix_sort_pairs(keys[0].data(), vals[0].data(), keys[1].data(), vals[1].data(), cnt.data(),
-                                         M, bits, hist, chunk, s);
+                                         M, bits, hist, s);
         reset_best_kernel<<<grid_p(V), kT, 0, s>>>(best.data(), target.data(), V);
         cbest_kernel<<<grid_p(M), kT, 0, s>>>(keys[cur].data(), M, V, szc, K, (uint32_t)round, best.data());
         ctarget_kernel<<<grid_p(M), kT, 0, s>>>(keys[cur].data(), M, V, szc, K, (uint32_t)round, best.data(),

@@ -147,6 +147,34 @@ def test_convert_runs_of_duplicates(ctx, dtype, runs):
     ls.close()
 
 
+@pytest.mark.parametrize("T,B", [(1, 1), (1024, 40), (4097, 700), (131072, 3000), (131073, 3000), (131072, 200000),
+                                 (700000, 200000)])
+def test_convert_sort_sizes(ctx, T, B):
+    """one tile of the radix sort, its small form's limit (131,072 keys) and one
+    key more, with 32-bit and (200,000 rows, any column) 64-bit keys, with
+    dropped triplets: BCOO bit for bit, and the product through the layout
+    built from the sorted lower entries"""
+    rng = np.random.default_rng(T + B)
+    r = rng.integers(0, B, T).astype(np.int32)
+    c = rng.integers(0, B, T).astype(np.int32)
+    drop = rng.random(T) < 0.1
+    rows = np.where(drop, -1, np.minimum(r, c)).astype(np.int32)
+    cols = np.maximum(r, c).astype(np.int32)
+    vals = rng.standard_normal((T, 9))
+    ls = LinearSystem(ctx, B)
+    ls.assemble(ctx.to_device(rows), ctx.to_device(cols), ctx.to_device(vals))
+    br, bc, bv, rp = ls.export_bcoo()
+    orr, oc, ov, orp = O.convert_sym(B, rows, cols, vals)
+    assert np.array_equal(br, orr) and np.array_equal(bc, oc) and np.array_equal(rp, orp)
+    assert np.array_equal(bv.view(np.uint64), ov.reshape(bv.shape).view(np.uint64))
+    x = rng.standard_normal(3 * B)
+    yref, _ = O.spmv_sym(B, orr, oc, ov, x)
+    yd = ctx.alloc(3 * B, np.float64)
+    ls.spmv(1.0, ctx.to_device(x), 0.0, yd)
+    assert np.abs(yd.numpy() - yref).max() <= 1e-13 * np.abs(yref).max()  # as test_spmv_dot
+    ls.close()
+
+
 def test_convert_empty_and_reassemble(ctx, c1):
     ls = LinearSystem(ctx, 10)
     z = ctx.alloc(1, np.int32)
