@@ -104,6 +104,9 @@ struct mi_sys
     } graph_key;
     bool graph_failed = false;
 
+    // small systems: the iterations in one cooperative launch
+    SmallPcgScratch small;
+
     // batched solves (mi_pcg_solve_batched): the tile table of the last
     // segmentation, per-system scalars, tile partials and their own graph
     struct Batch
@@ -1379,6 +1382,16 @@ void run_iteration(mi_sys* sys, double* x, bool bypass, const LocalPreconditione
     pcg_update_p(sc, partB, gB, sys->p.data(), sys->z.data(), n, p32, s);
 }
 
+// MI_PCG_SMALL=0 keeps small systems on the launches of run_iteration
+bool pcg_small_enabled()
+{
+    static const bool on = [] {
+        const char* e = std::getenv("MI_PCG_SMALL");
+        return !(e && std::string(e) == "0");
+    }();
+    return on;
+}
+
 void read_scalars(mi_sys* sys, hipStream_t s)
 {
     MI_HIP(hipMemcpyAsync(sys->h_sc, sys->d_sc, sizeof(PcgScalars), hipMemcpyDeviceToHost, s));
@@ -1582,7 +1595,55 @@ extern "C" int mi_pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pc
     key.bufs[9] = sys->p32.data();
     key.stream  = s;
 
-    while(done < total)
+    // a small system's iterations run in one launch (pcg_small.hip) when its
+    // preconditioner is one that it knows
+    bool     one_launch = o.use_graph && !ordered && pcg_small_enabled();
+    SmallPcg sm;
+    if(one_launch)
+    {
+        const BsrMatrix& A = sys->A;
+        sm.B               = A.B;
+        sm.fptr            = A.full_ptr.data();
+        sm.fcols           = A.fcols.data();
+        sm.use32           = use32_sys;
+        sm.fvals           = use32_sys ? (const void*)A.fvals32.data() : (const void*)A.fvals.data();
+        sm.fstride         = A.fstride;
+        sm.sc              = sys->d_sc;
+        sm.x               = xs;
+        sm.r               = sys->r.data();
+        sm.p               = sys->p.data();
+        sm.slots           = A.B;
+        one_launch         = !A.has_win && A.has_full && A.B <= kSmallRows;
+        if(one_launch && !bypass && !sys->pcs.empty())
+        {
+            if(fused)
+            {
+                sm.D       = fused->diag3_inverse();
+                sm.blk_off = fused->dof_offset / 3;
+                sm.blk_cnt = fused->dof_count / 3;
+            }
+            else
+                one_launch = sys->pcs.size() == 1 && sys->pcs[0]->small_pcg(sm);
+        }
+    }
+    while(one_launch && done < total)
+    {
+        if(!pcg_small_launch(sm, sys->small, total - done, s))
+            break;
+        read_scalars(sys, s);
+        MI_REQUIRE(!h.stalled, MI_ERR_HIP, "mi_pcg_solve: a wait between workgroups ran out");
+        MI_REQUIRE(std::isfinite(h.rz_new), MI_ERR_NONFINITE,
+                   "mi_pcg_solve: non-finite r^T z at iteration " + std::to_string(h.iter));
+        done = h.iter;
+        if(h.converged)
+        {
+            converged = true;
+            // the whole check intervals a captured block runs
+            done = std::min<int64_t>((h.conv_iter + gb - 1) / gb * gb, total);
+            break;
+        }
+    }
+    while(!converged && done < total)
     {
         int64_t blk       = std::min<int64_t>(gb, total - done);
         bool    use_graph = o.use_graph && !sys->graph_failed && blk == gb && s != nullptr;

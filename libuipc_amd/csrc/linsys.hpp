@@ -393,6 +393,7 @@ float  norm_f32_host(const float* x, int64_t n, hipStream_t s);
 // ----------------------------------------------------------------- preconditioners
 struct BatchScalars;
 struct PcgScalars;
+struct SmallPcg;
 // LocalPreconditioner (linear_system/local_preconditioner.h:9-49)
 class LocalPreconditioner
 {
@@ -424,6 +425,9 @@ class LocalPreconditioner
     // must be zero when it starts (the caller clears them in the x, r
     // update); 0 when apply_dot writes its partials without atomics
     virtual int dot_slots() const { return 0; }
+    // MAS only: its tables for the one-launch iterations of small systems
+    // (vectors in the caller's order); false when they cannot take it
+    virtual bool small_pcg(SmallPcg&) const { return false; }
     // MAS only: levels used by apply (MASPreconditionerEngine::set_active_level_num)
     virtual bool set_active_levels(int) { return false; }
     // MAS only, batched solves: a level count per system (block-row ranges)
@@ -473,6 +477,7 @@ struct PcgScalars
     int32_t criterion;
     int32_t iter;
     int32_t conv_iter;
+    int32_t stalled;  // a wait between workgroups ran out (pcg_small_launch)
 };
 
 // the fixed-order sum of a reduction's partials (stride apart), redone by every
@@ -641,6 +646,47 @@ void batch_alpha_xr(const BatchTiles& t, BatchScalars* sc, int32_t nseg, const d
                     const double* p, double* r, const double* Ap, hipStream_t s);
 void batch_beta_p(const BatchTiles& t, BatchScalars* sc, int32_t nseg, const double* rz, const double* rr,
                   double* p, const double* z, float4* p32, hipStream_t s);
+
+// ---- small systems: many iterations in one cooperative launch (pcg_small.hip)
+constexpr int kSmallRows = 16384;  // rows, and MAS partition slots, it takes
+struct SmallPcg
+{
+    // the full BSR
+    int32_t        B       = 0;
+    const int32_t* fptr    = nullptr;
+    const int32_t* fcols   = nullptr;
+    const void*    fvals   = nullptr;
+    int64_t        fstride = 0;
+    bool           use32   = false;  // float values
+    // the solve's state (read and written)
+    PcgScalars* sc = nullptr;
+    double *    x = nullptr, *r = nullptr, *p = nullptr;
+    // rows by slot: slots = B and slot_vec = null, or the MAS partition's
+    int32_t        slots    = 0;
+    const int32_t* slot_vec = nullptr;
+    // 3x3 block Jacobi (D null: the identity)
+    const double* D       = nullptr;
+    int64_t       blk_off = 0, blk_cnt = 0;
+    // MAS: inverses (9 planes per cluster), levels run, slots' parents, sibling
+    // masks and ancestors, coarse clusters and their nodes' descendants
+    const void*    inv    = nullptr;
+    bool           inv32  = false;
+    int32_t        levels = 1, coarse = 0;
+    int64_t        c_first = 0, c_desc = 0, nodes = 0;
+    const int32_t *parent = nullptr, *sib = nullptr, *anc_slot = nullptr, *desc_ptr = nullptr, *desc_idx = nullptr;
+    // filled by pcg_small_launch
+    uint64_t* words = nullptr;
+    double *  z = nullptr, *pb = nullptr, *R = nullptr, *RA = nullptr, *Z = nullptr;
+    int32_t   max_it = 0;
+};
+struct SmallPcgScratch
+{
+    DBuf<uint64_t> words;
+    DBuf<double>   z, pb, R, Z;
+};
+// up to max_it iterations from the state in `a`; false when this system, or
+// this device, cannot run them so (nothing is launched then)
+bool pcg_small_launch(SmallPcg& a, SmallPcgScratch& scr, int64_t max_it, hipStream_t s);
 
 // allocates the PCG reductions' partials (must run before any pointer into them is taken)
 void pcg_prepare(SpmvScratch& scr);

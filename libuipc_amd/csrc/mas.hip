@@ -2233,6 +2233,30 @@ class MasPreconditioner final : public LocalPreconditioner
         return true;
     }
 
+    // the whole vector in the caller's order, every vertex in a part, level 1
+    // the base of the coarser levels' sums
+    bool small_pcg(SmallPcg& a) const override
+    {
+        if(dof_offset != 0 || dof_count != 3 * (int64_t)a.B || n_unpart != 0 || fine_lvl || row_order_ || h.V == 0
+           || (h.L > 1 && base_lvl != 1))
+            return false;
+        a.slots    = h.N;
+        a.slot_vec = d_part_to_real.data();
+        a.inv      = fp32 ? (const void*)d_inv32.data() : (const void*)d_inv64.data();
+        a.inv32    = fp32 != 0;
+        a.levels   = levels_run();
+        a.c_first  = c_first;
+        a.coarse   = a.levels > 1 ? (int32_t)(C - c_first) : 0;
+        a.c_desc   = c_desc;
+        a.nodes    = h.total;
+        a.parent   = d_parent.data();
+        a.sib      = d_sib.data();
+        a.anc_slot = d_anc_slot.data();
+        a.desc_ptr = d_desc_ptr.data();
+        a.desc_idx = d_desc_idx.data();
+        return true;
+    }
+
     // fine clusters of stopped systems are skipped; the restriction and the
     // coarse levels (a few percent of the apply) still run over everything
     void skip_stopped(const int32_t* seg, int32_t nseg, const BatchScalars* sc, hipStream_t s) override

@@ -198,6 +198,7 @@ __global__ __launch_bounds__(kThreads) void pcg_init_scalars_kernel(PcgScalars* 
         sc->criterion  = criterion;
         sc->iter       = 0;
         sc->conv_iter  = 0;
+        sc->stalled    = 0;
     }
 }
 

@@ -1,0 +1,118 @@
+"""The PCG iterations of small systems in one cooperative launch
+(csrc/pcg_small.hip) against the launches of one iteration after another."""
+import numpy as np
+import pytest
+
+from libuipc_amd import abi, synth
+from libuipc_amd.device import LinearSystem, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def solve_both(ctx, ls, b, tol=1e-8, **kw):
+    """one launch (the default), and use_graph = 0: plain launches"""
+    out = []
+    for use_graph in (1, 0):
+        x = ctx.alloc(ls.n, np.float64)
+        if "x_init" in kw:
+            x.upload(kw["x0"])
+        opts = {k: v for k, v in kw.items() if k != "x0"}
+        st = ls.solve(b, x, tol=tol, use_graph=use_graph, true_residual=1, **opts)
+        out.append((st, x.numpy()))
+    return out
+
+
+def check(ctx, ls, b, tol=1e-8, err=1e-6, **kw):
+    (s1, x1), (s0, x0) = solve_both(ctx, ls, b, tol, criterion=abi.MI_CRIT_REL_RESIDUAL, **kw)
+    assert s1["converged"] == s0["converged"] == 1
+    # rounding moves a stiff system's count: at most 10% more, the bound of
+    # test_mas_pcg (with float inverses it takes up to 20% fewer: the launches
+    # restrict and add in float, this in double)
+    assert s1["iters_exact"] <= max(s0["iters_exact"] + 2, 1.1 * s0["iters_exact"])
+    # a float matrix leaves a residual of its rounding times the first residual,
+    # which both have; CG's rounding spreads it by a small factor
+    assert s1["rel_res_true"] < max(1e-7, 3.0 * s0["rel_res_true"])
+    assert rel_err(x1, x0) < err
+
+
+def dense_spd(B, per_row, seed):
+    """a block-diagonally dominant system with about 2 per_row random blocks in a row"""
+    rng = np.random.default_rng(seed)
+    r = np.repeat(np.arange(B), per_row)
+    c = rng.integers(0, B, r.size)
+    lo, hi = np.minimum(r, c), np.maximum(r, c)
+    off = lo != hi
+    lo, hi = lo[off], hi[off]
+    v = rng.standard_normal((lo.size, 9))
+    rows = np.concatenate([np.arange(B), lo]).astype(np.int32)
+    cols = np.concatenate([np.arange(B), hi]).astype(np.int32)
+    diag = np.tile(np.eye(3).ravel() * 14.0 * per_row, (B, 1))
+    return rows, cols, np.concatenate([diag, v])
+
+
+@pytest.mark.parametrize("B,per_row", [(1, 1), (63, 4), (64, 4), (65, 4), (700, 20), (2500, 60), (5000, 130), (16384, 6)])
+def test_small_pcg_rows(ctx, B, per_row):
+    """one row, workgroups one row short of and past 64 rows, blocks past the
+    registers (3,072 per workgroup) and columns past LDS (2,048), and the most
+    rows it takes"""
+    rows, cols, vals = dense_spd(B, per_row, seed=B)
+    ls = LinearSystem(ctx, B)
+    ls.assemble(ctx.to_device(rows), ctx.to_device(cols), ctx.to_device(vals))
+    b = ctx.to_device(np.random.default_rng(1).standard_normal(3 * B))
+    ls.add_preconditioner(abi.MI_PRECOND_DIAG3, 0, 3 * (B // 2))  # z = r on the other rows
+    ls.assemble_preconditioners()
+    check(ctx, ls, b)
+    ls.close()
+
+
+@pytest.mark.parametrize("precision,mas", [(abi.MI_FP64, abi.MI_FP64), (abi.MI_FP64, abi.MI_FP32),
+                                           (abi.MI_FP32, abi.MI_FP32)])
+@pytest.mark.parametrize("grid,contacts,levels", [(2, 0, 0), (5, 40, 0), (9, 900, 0), (9, 900, 1), (9, 900, 2),
+                                                  (17, 2000, 0), (25, 0, 0)])
+def test_small_pcg_mas(ctx, grid, contacts, levels, precision, mas):
+    """MAS over the whole vector at every kind of hierarchy (one cluster to six
+    levels), every level count, float and double storage"""
+    s = synth.fem_system(grid, contacts, seed=grid + 1)
+    ls = LinearSystem(ctx, s.block_rows, precision)
+    ls.assemble(ctx.to_device(s.rows), ctx.to_device(s.cols), ctx.to_device(s.vals))
+    ls.add_preconditioner(abi.MI_PRECOND_MAS, 0, s.n, part_ids=s.part_ids, tets=s.tets, mas_precision=mas,
+                          active_levels=levels)
+    ls.assemble_preconditioners()
+    b = ctx.to_device(s.rhs)
+    # contacts of four decades of stiffness: x to the residual times the condition
+    check(ctx, ls, b, err=1e-3)
+    # from a given x0, and the rz criterion
+    x0 = np.random.default_rng(3).standard_normal(s.n)
+    check(ctx, ls, b, err=1e-3, x_init=1, x0=x0)
+    ls.close()
+
+
+def test_small_pcg_stops(ctx):
+    """the iteration cap, the interval counts and a NaN in b, as the launches"""
+    s = synth.fem_system(9, 900, seed=2)
+    ls = LinearSystem(ctx, s.block_rows)
+    ls.assemble(ctx.to_device(s.rows), ctx.to_device(s.cols), ctx.to_device(s.vals))
+    ls.add_preconditioner(abi.MI_PRECOND_DIAG3, 0, s.n)
+    ls.assemble_preconditioners()
+    b = ctx.to_device(s.rhs)
+    for cap in (7.5, 530.5):  # within one launch and past its 512 iterations
+        (s1, x1), (s0, x0) = solve_both(ctx, ls, b, criterion=abi.MI_CRIT_REL_RESIDUAL, tol=1e-12,
+                                        max_iter_ratio=cap / s.n)
+        assert [s1[k] for k in ("iters", "converged")] == [s0[k] for k in ("iters", "converged")] == [int(cap), 0]
+        # up to 530 iterations of a stiff system, where rounding differences grow
+        assert rel_err(x1, x0) < 1e-3
+    # without contacts the counts do not depend on rounding
+    free = synth.fem_system(9, 0, seed=2)
+    lf = LinearSystem(ctx, free.block_rows)
+    lf.assemble(ctx.to_device(free.rows), ctx.to_device(free.cols), ctx.to_device(free.vals))
+    for ci in (1, 7):
+        (s1, x1), (s0, x0) = solve_both(ctx, lf, ctx.to_device(free.rhs), tol=1e-6, check_interval=ci)
+        assert [s1[k] for k in ("iters", "iters_exact")] == [s0[k] for k in ("iters", "iters_exact")]
+        assert rel_err(x1, x0) < 1e-9
+    lf.close()
+    bad = s.rhs.copy()
+    bad[5] = np.nan
+    with pytest.raises(abi.MiError) as e:
+        ls.solve(ctx.to_device(bad), ctx.alloc(s.n, np.float64))
+    assert e.value.code == abi.MI_ERR_NONFINITE
+    ls.close()
