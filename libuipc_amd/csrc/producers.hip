@@ -22,7 +22,7 @@
 // writer does (utils/matrix_assembler.h:312-437): slot (a, b), a <= b, in the
 // order a = 0..3, b = a..3; the block is written at (min, max) of the two
 // global vertex ids, transposed when the stencil order is reversed.
-// One thread per tet / stencil / vertex; all arithmetic in FP64.
+// All arithmetic in FP64.
 #include "linsys.hpp"
 
 namespace mi
@@ -153,28 +153,74 @@ __device__ void svd3(const double F[9], double U[9], double S[3], double V[9])
     S[2] = U[6] * Fv[2][0] + U[7] * Fv[2][1] + U[8] * Fv[2][2];
 }
 
-// writes slot (a, b) of a 4-node stencil: (min, max) of the global ids, the
-// block transposed when the stencil order is reversed; K_ab is row-major
-__device__ __forceinline__ void emit_block(const int32_t idx[4],
-                                           int           a,
-                                           int           b,
-                                           const double  K[3][3],
-                                           int64_t       t,
-                                           int32_t*      rows,
-                                           int32_t*      cols,
-                                           double*       vals)
+// The triplets of 4-node stencils, written by consecutive lanes: a stencil's 10
+// blocks are 720 consecutive bytes, which one lane per stencil writes in 90
+// stores that each touch 64 cache lines per wave.  Instead a wave's 64 stencils
+// pass each slot's blocks through LDS and nine lanes write a block
+// (StencilOut), or every lane computes the consecutive entries it writes
+// (contact_kernel).
+constexpr int kSlots = 10;
+// slot s = (a, b), a <= b: two bits per slot
+__device__ __forceinline__ constexpr int slot_a(int s)
 {
-    const bool swap = idx[a] > idx[b];
-    rows[t]         = swap ? idx[b] : idx[a];
-    cols[t]         = swap ? idx[a] : idx[b];
-    double* v       = vals + 9 * t;
-#pragma unroll
-    for(int c = 0; c < 3; ++c)
-#pragma unroll
-        for(int r = 0; r < 3; ++r)
-            v[r + 3 * c] = swap ? K[c][r] : K[r][c];
+    return (0xE9500 >> (2 * s)) & 3;  // 0 0 0 0 1 1 1 2 2 3
+}
+__device__ __forceinline__ constexpr int slot_b(int s)
+{
+    return (0xFB9E4 >> (2 * s)) & 3;  // 0 1 2 3 1 2 3 2 3 3
 }
 
+// rows and cols of n stencils (ids: LDS, 4 per stencil), by NT threads:
+// (min, max) of the slot's two ids
+template <int NT>
+__device__ __forceinline__ void put_ids(const int32_t (*ids)[4], int n, int t, int32_t* rows, int32_t* cols)
+{
+    for(int e = t; e < kSlots * n; e += NT)
+    {
+        const int     i = e / kSlots, s = e - kSlots * i;
+        const int32_t x = ids[i][slot_a(s)], y = ids[i][slot_b(s)];
+        rows[e]         = x < y ? x : y;
+        cols[e]         = x < y ? y : x;
+    }
+}
+
+// orders a wave's LDS accesses before it against those after it
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// one wave's stencils, a lane each: blocks of one slot at a time
+struct StencilOut
+{
+    double (*st)[9];       // LDS, one block per lane
+    int32_t (*ids)[4];     // LDS, the stencils' global ids
+    double* vals;          // of the wave's first stencil
+    int     n;             // its stencils
+    int     lane;
+    // K_ab row-major; written transposed when the stencil order is reversed
+    __device__ __forceinline__ void put(int s, const double K[3][3])
+    {
+        const bool swap = ids[lane][slot_a(s)] > ids[lane][slot_b(s)];
+#pragma unroll
+        for(int c = 0; c < 3; ++c)
+#pragma unroll
+            for(int r = 0; r < 3; ++r)
+                st[lane][r + 3 * c] = swap ? K[c][r] : K[r][c];
+        wave_lds_fence();
+#pragma unroll 1  // (unrolled, its addresses take 60 registers over the whole kernel)
+        for(int k = 0; k < 9; ++k)
+        {
+            const int e = k * kWave + lane, i = e / 9, q = e - 9 * i;
+            if(i < n)
+                vals[9 * (kSlots * i + s) + q] = st[i][q];
+        }
+        wave_lds_fence();  // st is rewritten by the next slot
+    }
+};
+
+// one thread per entry: consecutive lanes write consecutive doubles
 __global__ __launch_bounds__(kThreads) void kinetic_kernel(int32_t V,
                                                           const double* __restrict__ mass,
                                                           int32_t  vert_offset,
@@ -182,18 +228,24 @@ __global__ __launch_bounds__(kThreads) void kinetic_kernel(int32_t V,
                                                           int32_t* cols,
                                                           double*  vals)
 {
-    for(int32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < V; v += gridDim.x * blockDim.x)
+    const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    for(int64_t i = i0; i < 9 * (int64_t)V; i += stride)
     {
-        rows[v]   = v + vert_offset;
-        cols[v]   = v + vert_offset;
-        double* o = vals + 9 * (int64_t)v;
-#pragma unroll
-        for(int q = 0; q < 9; ++q)
-            o[q] = (q % 4 == 0) ? mass[v] : 0.0;
+        const int64_t v = i / 9;
+        const int     q = (int)(i - 9 * v);
+        vals[i]         = q % 4 == 0 ? mass[v] : 0.0;
+    }
+    for(int64_t v = i0; v < V; v += stride)
+    {
+        rows[v] = (int32_t)v + vert_offset;
+        cols[v] = (int32_t)v + vert_offset;
     }
 }
 
-__global__ __launch_bounds__(kThreads) void snh_kernel(int64_t n_tets,
+// Bound by the registers of its FP64 arithmetic (two SVD-sized Jacobi sweeps)
+// and by the writes: 149k tets of a 32^3 grid 82 -> 51 us (119 MB written) with
+// three waves per SIMD (four: 128 registers and 146 us of spills; one, of 256: 63).
+__global__ __launch_bounds__(kThreads, 3) void snh_kernel(int64_t n_tets,
                                                       const int32_t* __restrict__ tets,
                                                       const double* __restrict__ X,
                                                       const double* __restrict__ x,
@@ -205,16 +257,25 @@ __global__ __launch_bounds__(kThreads) void snh_kernel(int64_t n_tets,
                                                       int32_t* cols,
                                                       double*  vals)
 {
-    for(int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n_tets; t += (int64_t)gridDim.x * blockDim.x)
+    __shared__ double  st[kThreads][9];
+    __shared__ int32_t ids[kThreads][4];
+    const int          lane = threadIdx.x % kWave, w0 = threadIdx.x - lane;
+    // a wave's 64 tets in a row; lanes past the last repeat it and write nothing
+    for(int64_t t0 = (int64_t)blockIdx.x * kThreads + w0; t0 < n_tets; t0 += (int64_t)gridDim.x * kThreads)
     {
-        int32_t q[4], idx[4];
+        const int     n = n_tets - t0 < kWave ? (int)(n_tets - t0) : kWave;
+        const int64_t t = t0 + (lane < n ? lane : n - 1);
+        int32_t       q[4];
 #pragma unroll
         for(int c = 0; c < 4; ++c)
         {
-            q[c]   = tets[4 * t + c];
-            idx[c] = q[c] + vert_offset;
+            q[c]                 = tets[4 * t + c];
+            ids[threadIdx.x][c] = q[c] + vert_offset;
         }
-        double Dm[9], Ds[9], Dmi[9], F[9];
+        wave_lds_fence();
+        put_ids<kWave>(&ids[w0], n, lane, rows + kSlots * t0, cols + kSlots * t0);
+        StencilOut out{&st[w0], &ids[w0], vals + 9 * kSlots * t0, n, lane};
+        double     Dm[9], Ds[9], Dmi[9], F[9];
 #pragma unroll
         for(int c = 0; c < 3; ++c)
 #pragma unroll
@@ -264,66 +325,77 @@ __global__ __launch_bounds__(kThreads) void snh_kernel(int64_t n_tets,
         A[0][2] = A[2][0] = c2 * S[1];
         A[1][2] = A[2][1] = c2 * S[0];
         jacobi3(A, ew, ev);
-        // the 10 upper blocks, each summed over the 9 modes: lam w_a w_b^T
-        constexpr int kPairs[3][2] = {{1, 2}, {0, 2}, {0, 1}};  // (i, j) of the mode with third index k
-        const double  r2           = 0.70710678118654752440;  // 1 / sqrt(2)
-        int64_t       slot         = 10 * t;
+        // The 10 upper blocks, K_ab = U T_ab U^T with T_ab in the frame of the
+        // singular vectors: the scaling modes' projected Hessian P couples sa_i
+        // and sb_j, the twist and flip modes of a pair (i, j) (eigenvalues lt, lf
+        // with the vectors (U_i s_j -/+ U_j s_i) / sqrt 2) give (lt + lf) / 2 on
+        // the diagonal and (lf - lt) / 2 off it.  (Summing lam w_a w_b^T over
+        // the nine modes is five times the arithmetic.)
+        double P[3][3], ht[3], hd[3];
+#pragma unroll
+        for(int i = 0; i < 3; ++i)
+#pragma unroll
+            for(int j = i; j < 3; ++j)
+            {
+                double acc = 0.0;
+#pragma unroll
+                for(int m = 0; m < 3; ++m)
+                    acc += fmax(ew[m], 0.0) * (ev[i][m] * ev[j][m]);
+                P[i][j] = P[j][i] = scale * acc;
+            }
+#pragma unroll
+        for(int k = 0; k < 3; ++k)
+        {
+            const double lt = fmax(mu + s * S[k], 0.0), lf = fmax(mu - s * S[k], 0.0);
+            ht[k]           = 0.5 * scale * (lt + lf);
+            hd[k]           = 0.5 * scale * (lf - lt);
+        }
+        int slot = 0;
 #pragma unroll
         for(int a = 0; a < 4; ++a)
 #pragma unroll
             for(int b = a; b < 4; ++b)
             {
-                double K[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-                // scaling modes: w_i = U (e_m (.) sa_i)
+                double pr[3][3];  // sa_i sb_j
 #pragma unroll
-                for(int m = 0; m < 3; ++m)
-                {
-                    const double l = fmax(ew[m], 0.0) * scale;
-                    double       wa[3], wb[3];
+                for(int i = 0; i < 3; ++i)
 #pragma unroll
-                    for(int r = 0; r < 3; ++r)
-                    {
-                        wa[r] = U[r] * ev[0][m] * sa[a][0] + U[r + 3] * ev[1][m] * sa[a][1]
-                                + U[r + 6] * ev[2][m] * sa[a][2];
-                        wb[r] = U[r] * ev[0][m] * sa[b][0] + U[r + 3] * ev[1][m] * sa[b][1]
-                                + U[r + 6] * ev[2][m] * sa[b][2];
-                    }
+                    for(int j = 0; j < 3; ++j)
+                        pr[i][j] = sa[a][i] * sa[b][j];
+                double T[3][3];
 #pragma unroll
-                    for(int r = 0; r < 3; ++r)
+                for(int i = 0; i < 3; ++i)
 #pragma unroll
-                        for(int c = 0; c < 3; ++c)
-                            K[r][c] += l * wa[r] * wb[c];
-                }
-                // twist (-) and flip (+) modes of the pair (i, j), third index k:
-                // w = (U_i sa[j] -/+ U_j sa[i]) / sqrt(2)
-#pragma unroll
-                for(int k = 0; k < 3; ++k)
-                {
-                    const int i = kPairs[k][0], j = kPairs[k][1];
-#pragma unroll
-                    for(int flip = 0; flip < 2; ++flip)
-                    {
-                        const double l  = fmax(flip ? mu - s * S[k] : mu + s * S[k], 0.0) * scale;
-                        const double sg = flip ? 1.0 : -1.0;
-                        double       wa[3], wb[3];
-#pragma unroll
-                        for(int r = 0; r < 3; ++r)
+                    for(int j = 0; j < 3; ++j)
+                        if(i == j)
                         {
-                            wa[r] = r2 * (U[r + 3 * i] * sa[a][j] + sg * U[r + 3 * j] * sa[a][i]);
-                            wb[r] = r2 * (U[r + 3 * i] * sa[b][j] + sg * U[r + 3 * j] * sa[b][i]);
+                            const int u = (i + 1) % 3, v = (i + 2) % 3;  // pairs (i, u) and (i, v): third indices v, u
+                            T[i][i] = P[i][i] * pr[i][i] + ht[v] * pr[u][u] + ht[u] * pr[v][v];
                         }
+                        else
+                            T[i][j] = P[i][j] * pr[i][j] + hd[3 - i - j] * pr[j][i];
+                double UT[3][3], K[3][3];
 #pragma unroll
-                        for(int r = 0; r < 3; ++r)
+                for(int r = 0; r < 3; ++r)
 #pragma unroll
-                            for(int c = 0; c < 3; ++c)
-                                K[r][c] += l * wa[r] * wb[c];
-                    }
-                }
-                emit_block(idx, a, b, K, slot++, rows, cols, vals);
+                    for(int j = 0; j < 3; ++j)
+                        UT[r][j] = U[r] * T[0][j] + U[r + 3] * T[1][j] + U[r + 6] * T[2][j];
+#pragma unroll
+                for(int r = 0; r < 3; ++r)
+#pragma unroll
+                    for(int c = 0; c < 3; ++c)
+                        if(a == b && c < r)
+                            K[r][c] = K[c][r];  // a diagonal block is symmetric to the bit
+                        else
+                            K[r][c] = UT[r][0] * U[c] + UT[r][1] * U[c + 3] + UT[r][2] * U[c + 6];
+                out.put(slot++, K);
             }
     }
 }
 
+// A workgroup takes 64 stencils at a time: their g, kappa and ids staged in LDS,
+// then every lane computes the consecutive entries it writes.  Bound by them:
+// 200k stencils (160 MB written, 21 MB read) 76 -> 42 us, 4.3 TB/s.
 __global__ __launch_bounds__(kThreads) void contact_kernel(int64_t n,
                                                           const int32_t* __restrict__ cidx,
                                                           const double* __restrict__ g,
@@ -334,37 +406,32 @@ __global__ __launch_bounds__(kThreads) void contact_kernel(int64_t n,
                                                           int32_t* cols,
                                                           double*  vals)
 {
-    for(int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; s < n; s += (int64_t)gridDim.x * blockDim.x)
+    constexpr int      kN = 64;
+    __shared__ double  sg[kN][12], sk[kN];
+    __shared__ int32_t ids[kN][4];
+    const int          tid = threadIdx.x;
+    for(int64_t s0 = (int64_t)blockIdx.x * kN; s0 < n; s0 += (int64_t)gridDim.x * kN)
     {
-        int32_t idx[4];
-#pragma unroll
-        for(int c = 0; c < 4; ++c)
-            idx[c] = cidx[4 * s + c] + vert_offset;
-        double gv[12];
-#pragma unroll
-        for(int c = 0; c < 12; ++c)
-            gv[c] = g[12 * s + c];
-        const double k    = dt2 * kappa[s];
-        int64_t      slot = 10 * s;
-#pragma unroll
-        for(int a = 0; a < 4; ++a)
-#pragma unroll
-            for(int b = a; b < 4; ++b)
-            {
-                // the block in its written orientation (L, R) = (a, b) or (b, a),
-                // each entry k g_(L, r) g_(R, c) as one product chain
-                const bool swap = idx[a] > idx[b];
-                const int  L = swap ? b : a, R = swap ? a : b;
-                rows[slot]   = idx[L];
-                cols[slot]   = idx[R];
-                double* v    = vals + 9 * slot;
-#pragma unroll
-                for(int c = 0; c < 3; ++c)
-#pragma unroll
-                    for(int r = 0; r < 3; ++r)
-                        v[r + 3 * c] = k * gv[3 * L + r] * gv[3 * R + c];
-                ++slot;
-            }
+        const int m = n - s0 < kN ? (int)(n - s0) : kN;
+        for(int e = tid; e < 12 * m; e += kThreads)
+            (&sg[0][0])[e] = g[12 * s0 + e];
+        if(tid < 4 * m)
+            (&ids[0][0])[tid] = cidx[4 * s0 + tid] + vert_offset;
+        if(tid < m)
+            sk[tid] = dt2 * kappa[s0 + tid];
+        __syncthreads();
+        put_ids<kThreads>(ids, m, tid, rows + kSlots * s0, cols + kSlots * s0);
+        for(int e = tid; e < 9 * kSlots * m; e += kThreads)
+        {
+            const int i = e / (9 * kSlots), f = e - 9 * kSlots * i, s = f / 9, q = f - 9 * s;
+            const int a = slot_a(s), b = slot_b(s);
+            // the block in its written orientation (L, R) = (a, b) or (b, a),
+            // each entry k g_(L, r) g_(R, c) as one product chain
+            const bool swap                = ids[i][a] > ids[i][b];
+            const int  L = swap ? b : a, R = swap ? a : b, c = q / 3, r = q - 3 * c;
+            vals[9 * kSlots * s0 + e]      = sk[i] * sg[i][3 * L + r] * sg[i][3 * R + c];
+        }
+        __syncthreads();
     }
 }
 // ---- line-search side: energies and the trial step
@@ -503,7 +570,7 @@ void produce_kinetic(int32_t V, const double* mass, int32_t vert_offset, int32_t
                      hipStream_t s)
 {
     if(V > 0)
-        kinetic_kernel<<<grid_of(V), kThreads, 0, s>>>(V, mass, vert_offset, rows, cols, vals);
+        kinetic_kernel<<<grid_of(9 * (int64_t)V), kThreads, 0, s>>>(V, mass, vert_offset, rows, cols, vals);
     MI_HIP(hipGetLastError());
 }
 
@@ -538,7 +605,7 @@ void produce_contact(int64_t        n,
                      hipStream_t    s)
 {
     if(n > 0)
-        contact_kernel<<<grid_of(n), kThreads, 0, s>>>(n, stencils, g, kappa, dt * dt, vert_offset, rows, cols, vals);
+        contact_kernel<<<grid_of(4 * n), kThreads, 0, s>>>(n, stencils, g, kappa, dt * dt, vert_offset, rows, cols, vals);
     MI_HIP(hipGetLastError());
 }
 }  // namespace mi

@@ -98,3 +98,36 @@ def test_produced_system_solves_like_the_host_one(ctx):
     assert d < 1e-6, d
     a.close()
     h.close()
+
+
+@pytest.mark.parametrize("grid,contacts", [(2, 1), (4, 63), (4, 64), (4, 65), (6, 257)])
+def test_producers_ragged_waves(ctx, grid, contacts):
+    """5, 135 and 625 tets and stencil counts around a wave's 64: the waves' last
+    lanes write nothing of their own, and nothing past the last triplet"""
+    s = synth.fem_system(grid, contacts, seed=3)
+    p = synth.producer_inputs(grid, contacts, seed=3)
+    B, nt = s.block_rows, len(p.tets)
+    T = s.n_triplets
+    rows, cols = (ctx.to_device(np.full(T + 64, -7, np.int32)) for _ in range(2))
+    vals = ctx.to_device(np.full((T + 64, 9), -7.0))
+    keep = [ctx.to_device(a) for a in (p.mass, p.tets, p.rest_positions, p.positions, p.contact_idx, p.contact_g,
+                                       p.contact_kappa)]
+    m, te, X, x, ci, cg, ck = (k.ptr for k in keep)
+    lib = ctx.lib
+
+    def at(k):
+        return rows.ptr.value + 4 * k, cols.ptr.value + 4 * k, vals.ptr.value + 72 * k
+
+    check(lib.mi_produce_kinetic(ctx.h, B, m, 0, *at(0), None))
+    check(lib.mi_produce_snh(ctx.h, nt, te, X, x, p.mu, p.lam, p.dt, 0, *at(B), None))
+    check(lib.mi_produce_contact(ctx.h, contacts, ci, cg, ck, p.dt, 0, *at(B + 10 * nt), None))
+    ctx.synchronize()
+    r, c, v = rows.numpy(), cols.numpy(), vals.numpy()
+    assert np.array_equal(r[:T], s.rows) and np.array_equal(c[:T], s.cols)
+    assert (r[T:] == -7).all() and (c[T:] == -7).all() and (v[T:] == -7.0).all()
+    fem = slice(B, B + 10 * nt)
+    assert np.array_equal(v[:B], s.vals[:B]) and np.array_equal(v[B + 10 * nt:T], s.vals[B + 10 * nt:])
+    # the numerical projection against the analytic one, as above
+    assert np.abs(v[fem] - s.vals[fem]).max() < 1e-9 * np.abs(s.vals[fem]).max()
+    diag = v[fem].reshape(nt, 10, 9)[:, [0, 4, 7, 9]].reshape(-1, 3, 3)
+    assert np.array_equal(diag, diag.transpose(0, 2, 1))
