@@ -421,13 +421,48 @@ __device__ __forceinline__ void agg_atomic_add(double* hess, int64_t dst, const 
             atomic_add_f64(hess + dst + q, v[q]);
 }
 
+// The same into an LDS cluster (at: entry, -1: nothing; every lane calls it):
+// destinations that many lanes share are summed over the wave first, the rest
+// are plain LDS atomics (64 lanes on one address serialise, a sum is 9
+// chains of DPP adds)
+__device__ __forceinline__ void lds_add(double* cl, int32_t at, const double (&v)[9])
+{
+    bool pending = at >= 0;
+    for(;;)
+    {
+        const uint64_t act = __ballot(pending);
+        if(act == 0)
+            return;
+        const int      leader = __ffsll((long long)act) - 1;
+        const int32_t  la     = __builtin_amdgcn_readlane(at, leader);
+        const bool     mine   = pending && at == la;
+        const uint64_t peers  = __ballot(mine);
+        if(__popcll(peers) < 16)
+            break;
+#pragma unroll
+        for(int q = 0; q < 9; ++q)
+        {
+            const double s = wave_total(mine ? v[q] : 0.0);
+            if(__lane_id() == leader)
+                atomicAdd(&cl[la + q], s);
+        }
+        if(mine)
+            pending = false;
+    }
+    if(pending)
+#pragma unroll
+        for(int q = 0; q < 9; ++q)
+            atomicAdd(&cl[at + q], v[q]);
+}
+
 // One upper block (r, c) of the MAS's range (local rows, sr / sc their
 // partition slots; live = a block to walk, every lane of the wave calls this):
 // level 0 by a plain store (each cluster entry has this one source, scatter
 // k1, mas_preconditioner_engine.cu:530-682), the coarse levels' off-diagonal
 // in-bank contributions until the ancestors merge by wave-aggregated atomics
-// -- level 1 into the caller's LDS copy of its level-1 cluster instead when
-// l1 is given (lds_base: that cluster's first entry in hess).
+// -- into the caller's LDS copies of one cluster per coarse level when lc is
+// given (base[l - 1]: level l's first entry in hess; a contribution outside
+// them goes to memory).
 __device__ __forceinline__ void walk_block(bool           live,
                                            int64_t        u,
                                            int32_t        r,
@@ -439,8 +474,8 @@ __device__ __forceinline__ void walk_block(bool           live,
                                            const int32_t* __restrict__ anc,
                                            int            L,
                                            double*        hess,
-                                           double*        l1,
-                                           int64_t        lds_base)
+                                           double (*lc)[kCm],
+                                           const int64_t* base)
 {
     double H[9];
     if(live)
@@ -479,14 +514,24 @@ __device__ __forceinline__ void walk_block(bool           live,
             H[q] = 0.0;
     }
     // coarse levels: off-diagonal in-bank contributions until the ancestors merge
-    for(int l = 1; l < L; ++l)
+    // (all levels' ancestors loaded at once, off the chain of the levels)
+    int32_t aa[kMaxLvl - 1], bb[kMaxLvl - 1];
+#pragma unroll
+    for(int l = 1; l < kMaxLvl; ++l)
     {
+        aa[l - 1] = live && l < L ? anc[(int64_t)(l - 1) * V + r] : -1;
+        bb[l - 1] = live && l < L ? anc[(int64_t)(l - 1) * V + c] : -1;
+    }
+#pragma unroll
+    for(int l = 1; l < kMaxLvl; ++l)
+    {
+        if(l >= L)
+            break;
         int64_t dst = -1;
         double  v[9];
         if(live)
         {
-            int32_t a = anc[(int64_t)(l - 1) * V + r];
-            int32_t b = anc[(int64_t)(l - 1) * V + c];
+            const int32_t a = aa[l - 1], b = bb[l - 1];
             if(a < 0 || b < 0 || a == b)
                 live = false;
             else if(a / kBank == b / kBank)
@@ -517,19 +562,13 @@ __device__ __forceinline__ void walk_block(bool           live,
         }
         if(__ballot(live) == 0)
             break;
-        if(l == 1 && l1)
+        if(lc)
         {
-            // the workgroup's own level-1 cluster: LDS atomics (an entry
-            // outside it, which the build's check rules out, goes to memory)
-            const int64_t e = dst - lds_base;
-            if(dst >= 0 && e >= 0 && e < kCm)
-#pragma unroll
-                for(int q = 0; q < 9; ++q)
-                    atomicAdd(&l1[e + q], v[q]);
-            else if(dst >= 0)
-#pragma unroll
-                for(int q = 0; q < 9; ++q)
-                    atomic_add_f64(hess + dst + q, v[q]);
+            const int64_t e  = dst - base[l - 1];
+            const bool    in = dst >= 0 && e >= 0 && e < kCm;
+            lds_add(lc[l - 1], in ? (int32_t)e : -1, v);
+            if(__ballot(dst >= 0 && !in) != 0)
+                agg_atomic_add(hess, in ? -1 : dst, v);
         }
         else
             agg_atomic_add(hess, dst, v);
@@ -563,11 +602,11 @@ __global__ __launch_bounds__(256) void mas_walk_kernel(int64_t        U,
         sc   = real_to_part[c];
         live = sr >= 0 && sc >= 0;
     }
-    walk_block(live, u, r, c, sr, sc, vals, V, anc, L, hess, nullptr, 0);
+    walk_block(live, u, r, c, sr, sc, vals, V, anc, L, hess, nullptr, nullptr);
 }
 
 
-// One round of the push for four clusters, one per wave (k; live: a
+// One round of the push for one cluster per wave (k; live: a
 // cluster to do): the full sum of each group of its nodes that share a
 // parent -> the parent's diagonal block.  A parent in the cluster whose
 // entries start at hess[l1_base] is written to l1 (LDS) when l1 is given.
@@ -654,53 +693,97 @@ __global__ __launch_bounds__(256) void mas_push_kernel(int64_t        c_first,
     push_round(k, live, parent, hess, S, P, nullptr, 0);
 }
 
+// upper block index -> (row node a, column node b), a <= b (inverse of sym_index)
+__device__ __forceinline__ void sym_rc(int blk, int& a, int& b)
+{
+    int r = 0;
+#pragma unroll
+    for(int t = 1; t < kBank; ++t)
+        r += blk >= kBank * t - t * (t - 1) / 2 ? 1 : 0;
+    a = r;
+    b = blk - (kBank * r - r * (r - 1) / 2) + r;
+}
+
 // The same walk in the partition order, one workgroup per 256-slot range
 // whose parts make up one level-1 bank (the build checks this): every
 // contribution to that level-1 cluster comes from the range's own rows, so
 // the workgroup adds them in LDS and stores the cluster once, where the
-// block-order walk spent most of its time in global atomics at level 1.
-// Blocks are taken row by row (the upper blocks of each slot's vertex), each
-// exactly once, as in the block-order walk; the level-0 push of the range's
-// parts follows, into the same LDS cluster (the push kernel then starts at
-// level 1).
-__global__ __launch_bounds__(256) void mas_walk_range_kernel(const int32_t* __restrict__ row_ptr,  // upper BCOO, global rows
-                                                            const int32_t* __restrict__ cols,
-                                                            const double* __restrict__ vals,
-                                                            int32_t        blk_off,
-                                                            int32_t        V,
-                                                            const int32_t* __restrict__ part_to_real,
-                                                            const int32_t* __restrict__ real_to_part,
-                                                            const int32_t* __restrict__ anc,
-                                                            int            L,
-                                                            const int32_t* __restrict__ range_bank,
-                                                            int64_t        c1_first,
-                                                            int32_t        nslots,
-                                                            const int32_t* __restrict__ parent,
-                                                            double*        hess)
+// block-order walk spent most of its time in global atomics at level 1.  The
+// levels above: a range's rows have few ancestors there, so its contributions
+// fall in one cluster per level; those are added in LDS too and go to memory
+// by atomics once per range (an address at the top levels met an atomic per
+// wave of blocks before).  Blocks are taken row by row (the upper blocks of each
+// slot's vertex), each exactly once, as in the block-order walk; the level-0
+// push of the range's parts follows, into the same LDS cluster (the push kernel
+// then starts at level 1).  16 waves per workgroup: a range is 4,000 to 5,000
+// blocks, whose loads are a chain of four, and a system has no more than two to
+// four ranges per CU.
+constexpr int kWalkNT = 1024;
+__global__ __launch_bounds__(kWalkNT) void mas_walk_range_kernel(const int32_t* __restrict__ row_ptr,  // upper BCOO, global rows
+                                                                const int32_t* __restrict__ cols,
+                                                                const double* __restrict__ vals,
+                                                                int32_t        blk_off,
+                                                                int32_t        V,
+                                                                const int32_t* __restrict__ part_to_real,
+                                                                const int32_t* __restrict__ real_to_part,
+                                                                const int32_t* __restrict__ anc,
+                                                                int            L,
+                                                                const int32_t* __restrict__ range_bank,
+                                                                int64_t        c1_first,
+                                                                int32_t        nslots,
+                                                                const int32_t* __restrict__ parent,
+                                                                int            push_all,
+                                                                double*        hess)
 {
-    __shared__ double   l1[kCm];
+    constexpr int       kW = kWalkNT / kWave;
+    __shared__ double   lc[kMaxLvl - 1][kCm];
+    __shared__ int64_t  base[kMaxLvl - 1];
     __shared__ uint32_t off[256 + 1];
-    __shared__ uint32_t lds[256 / kWave + 1];
-    const int     t     = threadIdx.x;
-    const int32_t bank  = range_bank[blockIdx.x];
-    const int64_t base1 = (c1_first + (bank < 0 ? 0 : bank)) * kCm;
-    for(int k = t; k < kCm; k += 256)
-        l1[k] = 0.0;
+    __shared__ uint32_t lds[kW + 1];
+    __shared__ int32_t  rs[256], bs[256];
+    const int     t    = threadIdx.x;
+    const int32_t bank = range_bank[blockIdx.x];
+    if(bank < 0)
+        return;  // no vertex in the range
+    for(int l = 1; l < L; ++l)
+        for(int k = t; k < kCm; k += kWalkNT)
+            lc[l - 1][k] = 0.0;
     // the range's rows and their upper-block counts
-    const int32_t slot = blockIdx.x * 256 + t;
-    const int32_t r    = slot < nslots ? part_to_real[slot] : -1;
-    const int32_t b0   = r >= 0 ? row_ptr[blk_off + r] : 0;
-    const uint32_t cnt = r >= 0 ? (uint32_t)(row_ptr[blk_off + r + 1] - b0) : 0u;
-    uint32_t      total;
-    const uint32_t o = block_exclusive_scan<256>(cnt, lds, &total);  // its barriers also order the l1 zeros
-    off[t]           = o;
+    const int32_t  slot = blockIdx.x * 256 + t;
+    const int32_t  r    = t < 256 && slot < nslots ? part_to_real[slot] : -1;
+    const int32_t  b0   = r >= 0 ? row_ptr[blk_off + r] : 0;
+    const uint32_t cnt  = r >= 0 ? (uint32_t)(row_ptr[blk_off + r + 1] - b0) : 0u;
+    uint32_t       total;
+    const uint32_t o = block_exclusive_scan<kWalkNT>(cnt, lds, &total);  // its barriers also order the zeros
+    if(t < 256)
+    {
+        off[t] = o;
+        rs[t]  = r;
+        bs[t]  = b0;
+    }
     if(t == 0)
         off[256] = total;
-    __shared__ int32_t rs[256], bs[256];
-    rs[t] = r;
-    bs[t] = b0;
+    if(t < kWave)
+    {
+        // the clusters kept in LDS: level 1's, and the one that holds the first
+        // vertex's ancestor at each level above
+        int32_t v = -1;
+        for(int q = 0; q < 4; ++q)
+        {
+            const int32_t  sl  = blockIdx.x * 256 + q * kWave + t;
+            const int32_t  y   = sl < nslots ? part_to_real[sl] : -1;
+            const uint64_t has = __ballot(y >= 0);
+            if(v < 0 && has)
+                v = __builtin_amdgcn_readlane(y, __ffsll((long long)has) - 1);
+        }
+        if(t >= 1 && t < L)
+        {
+            const int32_t a = anc[(int64_t)(t - 1) * V + v];
+            base[t - 1]     = t == 1 ? (c1_first + bank) * kCm : (int64_t)(a < 0 ? 0 : a / kBank) * kCm;
+        }
+    }
     __syncthreads();
-    for(uint32_t i0 = 0; i0 < total; i0 += 256)
+    for(uint32_t i0 = 0; i0 < total; i0 += kWalkNT)
     {
         const uint32_t i    = i0 + t;
         bool           live = i < total;
@@ -718,9 +801,9 @@ __global__ __launch_bounds__(256) void mas_walk_range_kernel(const int32_t* __re
                 else
                     hi = mid - 1;
             }
-            rr = rs[lo];
-            u  = (int64_t)bs[lo] + (i - off[lo]);
-            c  = cols[u] - blk_off;
+            rr   = rs[lo];
+            u    = (int64_t)bs[lo] + (i - off[lo]);
+            c    = cols[u] - blk_off;
             live = c >= 0 && c < V;
         }
         if(live)
@@ -729,34 +812,52 @@ __global__ __launch_bounds__(256) void mas_walk_range_kernel(const int32_t* __re
             sc   = real_to_part[c];
             live = sr >= 0 && sc >= 0;
         }
-        walk_block(live, u, rr, c, sr, sc, vals, V, anc, L, hess, l1, base1);
+        walk_block(live, u, rr, c, sr, sc, vals, V, anc, L, hess, lc, base);
     }
     // the level-0 push of the range's 16 parts (whose clusters this workgroup
     // has just stored; the barriers order those stores before the reads):
     // each level-1 node's diagonal block, into the LDS cluster
-    __shared__ double  S[4][kBank][9];
-    __shared__ int32_t P[4][kBank];
+    __shared__ double  S[kW][kBank][9];
+    __shared__ int32_t P[kW][kBank];
     __syncthreads();
     const int64_t c0 = nslots / kBank;  // level-0 clusters
-    for(int round = 0; round < 4; ++round)
+    for(int round = 0; round < kBank / kW; ++round)
     {
-        const int64_t k = (int64_t)blockIdx.x * kBank + round * 4 + t / kWave;
-        push_round(k, k < c0, parent, hess, S, P, l1, base1);
+        const int64_t k = (int64_t)blockIdx.x * kBank + round * kW + t / kWave;
+        push_round(k, k < c0, parent, hess, S, P, lc[0], base[0]);
     }
-    if(bank >= 0)
-        for(int k = t; k < kCm; k += 256)
-            hess[base1 + k] = l1[k];
-}
-
-// upper block index -> (row node a, column node b), a <= b (inverse of sym_index)
-__device__ __forceinline__ void sym_rc(int blk, int& a, int& b)
-{
-    int r = 0;
-#pragma unroll
-    for(int t = 1; t < kBank; ++t)
-        r += blk >= kBank * t - t * (t - 1) / 2 ? 1 : 0;
-    a = r;
-    b = blk - (kBank * r - r * (r - 1) / 2) + r;
+    // with push_all (every range's ancestors lie in one cluster per level, checked
+    // at the build) the pushes above follow in LDS too: a push is linear, so each
+    // range pushes its own share and the shares meet in the atomics below
+    for(int l = 1; push_all && l + 1 < L; ++l)
+    {
+        const int64_t node0 = base[l - 1] / kCm * kBank;
+        for(int e = t; e < kCm; e += kWalkNT)
+        {
+            const int blk = e / 9, q = e - 9 * blk;
+            int       a, b;
+            sym_rc(blk, a, b);
+            const int32_t pa = parent[node0 + a];
+            if(pa < 0 || pa != parent[node0 + b])
+                continue;
+            const int i = q % 3, j = q / 3;
+            double    v = lc[l - 1][9 * blk + q];
+            if(a != b)
+                v += lc[l - 1][9 * blk + j + 3 * i];
+            if(v != 0.0)
+                atomicAdd(&lc[l][9 * sym_index(pa % kBank, pa % kBank) + q], v);
+        }
+        __syncthreads();
+    }
+    for(int k = t; k < kCm; k += kWalkNT)
+        hess[base[0] + k] = lc[0][k];
+    for(int l = 2; l < L; ++l)
+        for(int k = t; k < kCm; k += kWalkNT)
+        {
+            const double v = lc[l - 1][k];
+            if(v != 0.0)
+                atomic_add_f64(hess + base[l - 1] + k, v);
+        }
 }
 
 // one wave per cluster: symmetric Gauss-Jordan sweep in FP64 (lane = column;
@@ -1768,6 +1869,7 @@ class MasPreconditioner final : public LocalPreconditioner
     bool           r0_fused_ = false;  // the PCG's x, r update wrote level 1's R (update_xr)
     bool           r1_fused_ = false;  // ... and level 2's
     bool           l1_local_ = false;  // every level-1 bank's parts lie in one 256-slot range
+    bool           all_local_ = false;  // ... and its ancestors in one cluster at every level above
     DBuf<int32_t>  d_fine_on;          // per fine cluster: 1 while it holds a running system
     const int32_t* fine_on = nullptr;  // d_fine_on during a batched solve, else nullptr
     DBuf<int32_t>  d_fine_lvl;         // per fine cluster: its system's level count (set_system_levels)
@@ -1950,6 +2052,23 @@ class MasPreconditioner final : public LocalPreconditioner
             }
             if(l1_local_)
                 upload(d_range_bank, range_bank);
+            // and does every range have its ancestors in one cluster at each level
+            // above (the assembly then pushes all levels range by range)?
+            all_local_ = l1_local_;
+            for(int l = 2; l < L && all_local_; ++l)
+            {
+                std::vector<int32_t> at((size_t)std::max(1, ranges), -1);
+                for(int32_t slot = 0; slot < h.N && all_local_; ++slot)
+                {
+                    const int32_t v = h.part_to_real[slot];
+                    if(v < 0)
+                        continue;
+                    const int32_t a = anc[(size_t)(l - 1) * h.V + v], cl = a < 0 ? -2 : a / kBank;
+                    if(at[slot / 256] == -1)
+                        at[slot / 256] = cl;
+                    all_local_ = cl >= 0 && at[slot / 256] == cl;
+                }
+            }
         }
         d_hess.resize((size_t)std::max<int64_t>(1, C * kCm));
         if(fp32)
@@ -1989,10 +2108,10 @@ class MasPreconditioner final : public LocalPreconditioner
             }();
             range_walk = l1_local_ && !by_blocks;
             if(range_walk)
-                mas_walk_range_kernel<<<ceil_div(h.N, 256), 256, 0, s>>>(
+                mas_walk_range_kernel<<<ceil_div(h.N, 256), kWalkNT, 0, s>>>(
                     A.row_ptr.data(), A.cols.data(), A.vals.data(), blk_off, h.V, d_part_to_real.data(),
                     d_real_to_part.data(), d_anc.data(), h.L, d_range_bank.data(), c_first, h.N, d_parent.data(),
-                    d_hess.data());
+                    all_local_ ? 1 : 0, d_hess.data());
             else
                 mas_walk_kernel<<<ceil_div(A.U, 256), 256, 0, s>>>(A.U,
                                                                    A.rows.data(),
@@ -2005,8 +2124,8 @@ class MasPreconditioner final : public LocalPreconditioner
                                                                    h.L,
                                                                    d_hess.data());
         }
-        // (the partition-order walk has done level 0's push)
-        for(int l = range_walk ? 1 : 0; l + 1 < h.L; ++l)
+        // (the partition-order walk has done level 0's push, or all of them)
+        for(int l = !range_walk ? 0 : all_local_ ? h.L : 1; l + 1 < h.L; ++l)
         {
             auto [first, cnt] = level_clusters[l];
             if(cnt > 0)
