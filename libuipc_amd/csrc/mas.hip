@@ -606,93 +606,6 @@ __global__ __launch_bounds__(256) void mas_walk_kernel(int64_t        U,
 }
 
 
-// One round of the push for one cluster per wave (k; live: a
-// cluster to do): the full sum of each group of its nodes that share a
-// parent -> the parent's diagonal block.  A parent in the cluster whose
-// entries start at hess[l1_base] is written to l1 (LDS) when l1 is given.
-// Every thread of the workgroup calls this (it holds barriers).
-__device__ __forceinline__ void push_round(int64_t        k,
-                                           bool           live,
-                                           const int32_t* __restrict__ parent,
-                                           double*        hess,
-                                           double (*S)[kBank][9],
-                                           int32_t (*P)[kBank],
-                                           double*        l1,
-                                           int64_t        l1_base)
-{
-    const int w    = threadIdx.x / kWave;
-    const int lane = threadIdx.x % kWave;
-    if(lane < kBank)
-    {
-        P[w][lane] = live ? parent[k * kBank + lane] : -1;
-#pragma unroll
-        for(int q = 0; q < 9; ++q)
-            S[w][lane][q] = 0.0;
-    }
-    __syncthreads();
-    if(live)
-    {
-        for(int blk = lane; blk < kSym; blk += kWave)
-        {
-            // blk -> (a, b), a <= b
-            int a = 0, rem = blk;
-            while(rem >= kBank - a)
-            {
-                rem -= kBank - a;
-                ++a;
-            }
-            int     b  = a + rem;
-            int32_t pa = P[w][a];
-            if(pa < 0 || pa != P[w][b])
-                continue;
-            int rep = 0;
-            while(P[w][rep] != pa)
-                ++rep;
-            const double* M = hess + k * kCm + 9 * blk;
-            for(int i = 0; i < 3; ++i)
-                for(int j = 0; j < 3; ++j)
-                {
-                    double val = M[i + 3 * j];
-                    if(a != b)
-                        val += M[j + 3 * i];
-                    atomicAdd(&S[w][rep][i + 3 * j], val);
-                }
-        }
-    }
-    __syncthreads();
-    if(live && lane < kBank)
-    {
-        int32_t pa = P[w][lane];
-        bool    first = pa >= 0;
-        for(int q = 0; q < lane && first; ++q)
-            first = P[w][q] != pa;
-        if(first)
-        {
-            const int64_t d = (int64_t)(pa / kBank) * kCm + 9 * sym_index(pa % kBank, pa % kBank);
-            double*       D = (l1 && d >= l1_base && d < l1_base + kCm) ? l1 + (d - l1_base) : hess + d;
-#pragma unroll
-            for(int q = 0; q < 9; ++q)
-                D[q] = S[w][lane][q];
-        }
-    }
-    __syncthreads();  // S and P are reused by the next round
-}
-
-// push(level): for every level-`level` cluster (one wave each), the full sum of
-// each group of its nodes that share a parent -> the parent's diagonal block
-__global__ __launch_bounds__(256) void mas_push_kernel(int64_t        c_first,
-                                                      int64_t        c_count,
-                                                      const int32_t* __restrict__ parent,
-                                                      double*        hess)
-{
-    __shared__ double  S[4][kBank][9];
-    __shared__ int32_t P[4][kBank];
-    const int     w    = threadIdx.x / kWave;
-    const int64_t k    = c_first + (int64_t)blockIdx.x * 4 + w;
-    const bool    live = (int64_t)blockIdx.x * 4 + w < c_count;
-    push_round(k, live, parent, hess, S, P, nullptr, 0);
-}
-
 // upper block index -> (row node a, column node b), a <= b (inverse of sym_index)
 __device__ __forceinline__ void sym_rc(int blk, int& a, int& b)
 {
@@ -702,6 +615,85 @@ __device__ __forceinline__ void sym_rc(int blk, int& a, int& b)
         r += blk >= kBank * t - t * (t - 1) / 2 ? 1 : 0;
     a = r;
     b = blk - (kBank * r - r * (r - 1) / 2) + r;
+}
+
+// The push of cluster k by one wave (every lane calls it): the full sum of
+// each group of its nodes that share a parent -> the parent's diagonal block.  A
+// parent in the cluster whose entries start at hess[l1_base] is written to l1
+// (LDS) when l1 is given.  The lanes hold the cluster's 136 blocks (three each)
+// and sum a group over the wave; a bank has one parent where its nodes are
+// connected.  (LDS atomics on the parent's nine entries, which all 64 lanes hit
+// at once, took 57 of the walk's 150 us on 41^3 + 400k.)
+__device__ __forceinline__ void push_cluster(int64_t        k,
+                                             const int32_t* __restrict__ parent,
+                                             double*        hess,
+                                             double*        l1,
+                                             int64_t        l1_base)
+{
+    const int     lane = threadIdx.x % kWave;
+    const int32_t mine = lane < kBank ? parent[k * kBank + lane] : -1;
+    double        M[3][9];  // a lane's blocks, plus their transposes off the diagonal
+    int32_t       pb[3];    // the parent that both nodes of the block share, else -1
+#pragma unroll
+    for(int h = 0; h < 3; ++h)
+    {
+        const int blk = lane + kWave * h;
+        int       a = 0, b = 0;
+        sym_rc(blk < kSym ? blk : 0, a, b);
+        const int32_t pa = __shfl(mine, a, kWave), pc = __shfl(mine, b, kWave);
+        pb[h] = blk < kSym && pa == pc ? pa : -1;
+#pragma unroll
+        for(int q = 0; q < 9; ++q)
+            M[h][q] = 0.0;
+        if(pb[h] >= 0)
+        {
+            const double* B = hess + k * kCm + 9 * blk;
+            double        m[9];
+#pragma unroll
+            for(int q = 0; q < 9; ++q)
+                m[q] = B[q];
+#pragma unroll
+            for(int i = 0; i < 3; ++i)
+#pragma unroll
+                for(int j = 0; j < 3; ++j)
+                    M[h][i + 3 * j] = a != b ? m[i + 3 * j] + m[j + 3 * i] : m[i + 3 * j];
+        }
+    }
+    for(uint64_t todo = __ballot(mine >= 0); todo;)
+    {
+        const int32_t p = __builtin_amdgcn_readlane(mine, __ffsll((long long)todo) - 1);
+        todo &= ~__ballot(mine == p);
+        double s[9];
+#pragma unroll
+        for(int q = 0; q < 9; ++q)
+        {
+            double v = 0.0;
+#pragma unroll
+            for(int h = 0; h < 3; ++h)
+                v += pb[h] == p ? M[h][q] : 0.0;
+            s[q] = wave_total(v);
+        }
+        if(lane == 0)
+        {
+            const int64_t d = (int64_t)(p / kBank) * kCm + 9 * sym_index(p % kBank, p % kBank);
+            double*       D = (l1 && d >= l1_base && d < l1_base + kCm) ? l1 + (d - l1_base) : hess + d;
+#pragma unroll
+            for(int q = 0; q < 9; ++q)
+                D[q] = s[q];
+        }
+    }
+}
+
+// push(level): for every level-`level` cluster (one wave each), the full sum of
+// each group of its nodes that share a parent -> the parent's diagonal block
+__global__ __launch_bounds__(256) void mas_push_kernel(int64_t        c_first,
+                                                      int64_t        c_count,
+                                                      const int32_t* __restrict__ parent,
+                                                      double*        hess)
+{
+    const int64_t k = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave;
+    if(k < c_count)
+        push_cluster(c_first + k, parent, hess, nullptr, 0);
 }
 
 // The same walk in the partition order, one workgroup per 256-slot range
@@ -817,15 +809,11 @@ __global__ __launch_bounds__(kWalkNT) void mas_walk_range_kernel(const int32_t* 
     // the level-0 push of the range's 16 parts (whose clusters this workgroup
     // has just stored; the barriers order those stores before the reads):
     // each level-1 node's diagonal block, into the LDS cluster
-    __shared__ double  S[kW][kBank][9];
-    __shared__ int32_t P[kW][kBank];
     __syncthreads();
-    const int64_t c0 = nslots / kBank;  // level-0 clusters
-    for(int round = 0; round < kBank / kW; ++round)
-    {
-        const int64_t k = (int64_t)blockIdx.x * kBank + round * kW + t / kWave;
-        push_round(k, k < c0, parent, hess, S, P, lc[0], base[0]);
-    }
+    for(int64_t k = (int64_t)blockIdx.x * kBank + t / kWave;
+        k < std::min<int64_t>(nslots / kBank, (int64_t)(blockIdx.x + 1) * kBank); k += kW)
+        push_cluster(k, parent, hess, lc[0], base[0]);
+    __syncthreads();
     // with push_all (every range's ancestors lie in one cluster per level, checked
     // at the build) the pushes above follow in LDS too: a push is linear, so each
     // range pushes its own share and the shares meet in the atomics below
