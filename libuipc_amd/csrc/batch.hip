@@ -6,8 +6,8 @@
 //   the SpMV runs over the union (no block couples two systems);
 //   every dot is a per-system sum: the DoFs are cut into tiles of at most
 //     kTile DoFs that never cross a system boundary (a host-built table), one
-//     workgroup writes each tile's partial, and one wave per system sums its
-//     tiles in order (deterministic, no atomics);
+//     workgroup writes each tile's partial, and every wave that needs a
+//     system's sum adds its tiles in order (deterministic, no atomics);
 //   alpha, beta, the convergence test and the iteration cap are per system;
 //     a system that has converged or reached its cap stops changing;
 //   the x / r and p updates run tile by tile, each tile reading its system's
@@ -111,29 +111,14 @@ __global__ __launch_bounds__(kThreads) void batch_bypass_z_kernel(const BatchTil
     }
 }
 
-// alpha = rz / pAp per system (fused_update_xr's scalar)
-__global__ void batch_alpha_kernel(const BatchTiles tiles, BatchScalars* sc, int32_t nseg, const double* pap)
-{
-    const int32_t s = (int32_t)((blockIdx.x * blockDim.x + threadIdx.x) / kWave);
-    if(s >= nseg)
-        return;
-    const double v = wave_tiles(pap, 1, tiles.sys_tile[s], tiles.sys_tile[s + 1]);
-    if(__lane_id() == 0)
-    {
-        BatchScalars& q = sc[s];
-        if(q.stopped)
-        {
-            q.alpha = 0.0;
-            return;
-        }
-        q.pAp   = v;
-        q.rz    = q.rz_pending;
-        q.alpha = q.rz / v;
-    }
-}
-
+// alpha = rz / pAp per system (fused_update_xr's scalar), then x and r.  Every
+// wave sums its system's partials by itself, in the same order; the
+// system's first tile records the scalars (no tile reads those it writes).  A
+// kernel of its own for them was 4.7 us of an iteration's 139 (12 systems of 3e3 to
+// 1e5 DoFs), and so was beta's.
 __global__ __launch_bounds__(kThreads) void batch_update_xr_kernel(const BatchTiles tiles,
-                                                                  const BatchScalars* __restrict__ sc,
+                                                                  BatchScalars* sc,
+                                                                  const double* __restrict__ pap,
                                                                   double*       x,
                                                                   const double* __restrict__ p,
                                                                   double*       r,
@@ -141,10 +126,19 @@ __global__ __launch_bounds__(kThreads) void batch_update_xr_kernel(const BatchTi
 {
     for(int32_t t = blockIdx.x; t < tiles.n; t += gridDim.x)
     {
-        const BatchScalars& q = sc[tiles.sys[t]];
+        const int32_t g = tiles.sys[t];
+        BatchScalars& q = sc[g];
         if(q.stopped)
             continue;
-        const double  alpha = q.alpha;
+        const int32_t t0 = tiles.sys_tile[g];
+        const double  rz = q.rz_pending, v = wave_tiles(pap, 1, t0, tiles.sys_tile[g + 1]);
+        const double  alpha = rz / v;
+        if(t == t0 && threadIdx.x == 0)
+        {
+            q.pAp   = v;
+            q.rz    = rz;
+            q.alpha = alpha;
+        }
         const int64_t lo = tiles.lo[t], hi = tiles.lo[t + 1];
         for(int64_t i = lo + threadIdx.x; i < hi; i += kThreads)
         {
@@ -154,52 +148,50 @@ __global__ __launch_bounds__(kThreads) void batch_update_xr_kernel(const BatchTi
     }
 }
 
-// convergence, beta and the cap per system (the scalar node of fused_pcg)
-__global__ void batch_beta_kernel(const BatchTiles tiles, BatchScalars* sc, int32_t nseg, const double* rz,
-                                  const double* rr)
-{
-    const int32_t s = (int32_t)((blockIdx.x * blockDim.x + threadIdx.x) / kWave);
-    if(s >= nseg)
-        return;
-    const double z = wave_tiles(rz, 1, tiles.sys_tile[s], tiles.sys_tile[s + 1]);
-    const double e = wave_tiles(rr, 1, tiles.sys_tile[s], tiles.sys_tile[s + 1]);
-    if(__lane_id() == 0)
-    {
-        BatchScalars& q = sc[s];
-        if(q.stopped)
-            return;
-        bool conv = q.criterion == 0 ? (fabs(z) <= q.rz_tol) : (e <= q.rr_tol);
-        if(!isfinite(z) || !isfinite(e))
-            conv = false;
-        const int64_t it = q.iter + 1;
-        q.iter           = it;
-        q.rz_new         = z;
-        q.rr             = e;
-        q.beta           = z / q.rz;
-        q.rz_pending     = z;
-        if(conv)
-        {
-            q.converged = 1;
-            q.conv_iter = it;
-            q.stopped   = 1;
-        }
-        else if(it >= q.max_iter - 1 || !isfinite(z))
-            q.stopped = 1;  // the cap of max_iter - 1 iterations (linear_fused_pcg.cu:1994)
-    }
-}
-
+// convergence, beta and the cap per system (the scalar node of fused_pcg),
+// recorded by the system's first tile, and p = z + beta p.  A converged system's
+// p and a non-finite one's are left by every tile (the sums are the same in all),
+// so p stays finite; at the cap a tile may be before or after the first one's
+// mark, and that p is read by nothing that counts.
 __global__ __launch_bounds__(kThreads) void batch_update_p_kernel(const BatchTiles tiles,
-                                                                 const BatchScalars* __restrict__ sc,
+                                                                 BatchScalars* sc,
+                                                                 const double* __restrict__ rz,
+                                                                 const double* __restrict__ rr,
                                                                  double*       p,
                                                                  const double* __restrict__ z,
                                                                  float4*       p32)
 {
     for(int32_t t = blockIdx.x; t < tiles.n; t += gridDim.x)
     {
-        const BatchScalars& q = sc[tiles.sys[t]];
-        if(q.stopped)
+        const int32_t g = tiles.sys[t];
+        BatchScalars& q = sc[g];
+        if(__hip_atomic_load(&q.stopped, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
             continue;
-        const double  beta = q.beta;
+        const int32_t t0 = tiles.sys_tile[g], t1 = tiles.sys_tile[g + 1];
+        const double  rz_new = wave_tiles(rz, 1, t0, t1), rr_new = wave_tiles(rr, 1, t0, t1);
+        const double  beta = rz_new / q.rz;
+        bool          conv = q.criterion == 0 ? (fabs(rz_new) <= q.rz_tol) : (rr_new <= q.rr_tol);
+        if(!isfinite(rz_new) || !isfinite(rr_new))
+            conv = false;
+        if(t == t0 && threadIdx.x == 0)
+        {
+            const int64_t it = q.iter + 1;
+            q.iter           = it;
+            q.rz_new         = rz_new;
+            q.rr             = rr_new;
+            q.beta           = beta;
+            q.rz_pending     = rz_new;
+            if(conv)
+            {
+                q.converged = 1;
+                q.conv_iter = it;
+            }
+            // or the cap of max_iter - 1 iterations (linear_fused_pcg.cu:1994)
+            if(conv || it >= q.max_iter - 1 || !isfinite(rz_new))
+                __hip_atomic_store(&q.stopped, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if(conv || !isfinite(rz_new))
+            continue;
         const int64_t lo = tiles.lo[t], hi = tiles.lo[t + 1];
         if(p32)
         {
@@ -338,19 +330,17 @@ void batch_bypass_z(const BatchTiles& t, const BatchScalars* sc, const int32_t* 
     MI_HIP(hipGetLastError());
 }
 
-void batch_alpha_xr(const BatchTiles& t, BatchScalars* sc, int32_t nseg, const double* pap, double* x,
+void batch_alpha_xr(const BatchTiles& t, BatchScalars* sc, const double* pap, double* x,
                     const double* p, double* r, const double* Ap, hipStream_t s)
 {
-    batch_alpha_kernel<<<seg_grid(nseg), kThreads, 0, s>>>(t, sc, nseg, pap);
-    batch_update_xr_kernel<<<tile_grid(t), kThreads, 0, s>>>(t, sc, x, p, r, Ap);
+    batch_update_xr_kernel<<<tile_grid(t), kThreads, 0, s>>>(t, sc, pap, x, p, r, Ap);
     MI_HIP(hipGetLastError());
 }
 
-void batch_beta_p(const BatchTiles& t, BatchScalars* sc, int32_t nseg, const double* rz, const double* rr,
+void batch_beta_p(const BatchTiles& t, BatchScalars* sc, const double* rz, const double* rr,
                   double* p, const double* z, float4* p32, hipStream_t s)
 {
-    batch_beta_kernel<<<seg_grid(nseg), kThreads, 0, s>>>(t, sc, nseg, rz, rr);
-    batch_update_p_kernel<<<tile_grid(t), kThreads, 0, s>>>(t, sc, p, z, p32);
+    batch_update_p_kernel<<<tile_grid(t), kThreads, 0, s>>>(t, sc, rz, rr, p, z, p32);
     MI_HIP(hipGetLastError());
 }
 }  // namespace mi

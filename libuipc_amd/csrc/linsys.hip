@@ -1717,20 +1717,19 @@ namespace
 void run_batch_iteration(mi_sys* sys, double* x, hipStream_t s)
 {
     auto&         bt    = sys->batch;
-    const int32_t nseg  = (int32_t)bt.seg_rows.size() - 1;
     const bool    use32 = sys->desc.value_precision == MI_FP32;
     float4*       p32   = use32 && !sys->A.has_win ? sys->p32.data() : nullptr;
     // rows of stopped systems are skipped: their Ap is never read again
     spmv_full(sys->A, use32, sys->p.data(), p32, sys->Ap.data(), sys->spmv_scr.partials.data(), nullptr,
               sys->spmv_scr, s, bt.active.data(), bt.n_active.data());
     batch_tile_dot(bt.tiles, sys->p.data(), sys->Ap.data(), bt.part_a.data(), nullptr, s);
-    batch_alpha_xr(bt.tiles, bt.sc.data(), nseg, bt.part_a.data(), x, sys->p.data(), sys->r.data(), sys->Ap.data(),
+    batch_alpha_xr(bt.tiles, bt.sc.data(), bt.part_a.data(), x, sys->p.data(), sys->r.data(), sys->Ap.data(),
                    s);
     sys->apply_preconditioner(sys->r.data(), sys->z.data(), nullptr, s);
     if(bt.any_bypass)
         batch_bypass_z(bt.tiles, bt.sc.data(), nullptr, sys->r.data(), sys->z.data(), s);
     batch_tile_dot(bt.tiles, sys->r.data(), sys->z.data(), bt.part_a.data(), bt.part_b.data(), s);
-    batch_beta_p(bt.tiles, bt.sc.data(), nseg, bt.part_a.data(), bt.part_b.data(), sys->p.data(), sys->z.data(), p32,
+    batch_beta_p(bt.tiles, bt.sc.data(), bt.part_a.data(), bt.part_b.data(), sys->p.data(), sys->z.data(), p32,
                  s);
 }
 

@@ -595,7 +595,10 @@ __device__ __forceinline__ double pcg_alpha_of(PcgScalars* sc, const double* pap
 // ---- batched PCG: independent systems on consecutive block-row ranges
 // Tiles of at most kBatchTile DoFs (whole block rows) that never cross a
 // system boundary; every per-system sum runs over its tiles in order.
-constexpr int64_t kBatchTile = 3 * 1365;
+// 1,023 DoFs give each of a workgroup's lanes four: 12 systems of 3e3 to 1e5 DoFs are
+// 420 tiles (with 4,095, 105: fewer workgroups than CUs; the dots 6.3 -> 4.7 us, x and r
+// 8.7 -> 5.3 with alpha's sum in it)
+constexpr int64_t kBatchTile = 3 * 341;
 // ----------------------------------------------------------------- learned initial guess
 void ws_gemm(int32_t M, int32_t N, int32_t K, const float* A, int64_t sa_m, int64_t sa_k, const float* B,
              int64_t sb_k, int64_t sb_n, float* C, int64_t ldc, bool accumulate, const float* bias, bool relu,
@@ -642,9 +645,9 @@ void batch_init(const BatchTiles& t, BatchScalars* sc, int32_t nseg, const doubl
 // with flags == null of the running systems whose preconditioner is bypassed
 void batch_bypass_z(const BatchTiles& t, const BatchScalars* sc, const int32_t* flags, const double* r, double* z,
                     hipStream_t s);
-void batch_alpha_xr(const BatchTiles& t, BatchScalars* sc, int32_t nseg, const double* pap, double* x,
+void batch_alpha_xr(const BatchTiles& t, BatchScalars* sc, const double* pap, double* x,
                     const double* p, double* r, const double* Ap, hipStream_t s);
-void batch_beta_p(const BatchTiles& t, BatchScalars* sc, int32_t nseg, const double* rz, const double* rr,
+void batch_beta_p(const BatchTiles& t, BatchScalars* sc, const double* rz, const double* rr,
                   double* p, const double* z, float4* p32, hipStream_t s);
 
 // ---- small systems: many iterations in one cooperative launch (pcg_small.hip)

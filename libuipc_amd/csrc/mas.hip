@@ -1373,6 +1373,62 @@ __global__ __launch_bounds__(256) void mas_restrict_level_kernel(const double* _
     restrict_bank<T, kLevel0>(r, slot_vec, Rb, parent, sib, begin + x, x < cnt);
 }
 
+// Levels 0 and 1 in one launch where every level-1 bank's parts lie in one
+// 256-slot range (checked at the build): the workgroup's level-1 sums also go to
+// LDS, where its bank's siblings are summed (as mas_update_xr_restrict_kernel's)
+// (1.4e5 vertices: 5.1 us against 4.8 + 4.7 for a launch per level)
+template <typename T>
+__global__ __launch_bounds__(256) void mas_restrict2_kernel(const double* __restrict__ r,
+                                                           const int32_t* __restrict__ slot_vec,
+                                                           T*             Rb,
+                                                           const int32_t* __restrict__ parent,
+                                                           const int32_t* __restrict__ sib,
+                                                           int32_t        nslots,
+                                                           int32_t        begin1,
+                                                           int32_t        count1,
+                                                           const int32_t* __restrict__ range_bank,
+                                                           const int32_t* conv)
+{
+    if(conv && *conv != 0)
+        return;
+    __shared__ T  r1s[kBank][3];
+    const int32_t slot  = blockIdx.x * 256 + threadIdx.x;
+    const bool    live  = slot < nslots;
+    const int32_t bank1 = range_bank[blockIdx.x];
+    const int32_t v     = live ? slot_vec[slot] : -1;
+    const int32_t m     = live ? sib[slot] : 0;
+    const int32_t par   = live ? parent[slot] : 0;
+    if(threadIdx.x < kBank)
+        r1s[threadIdx.x][0] = r1s[threadIdx.x][1] = r1s[threadIdx.x][2] = T(0);
+    T v0 = 0, v1 = 0, v2 = 0;
+    if(v >= 0)
+    {
+        v0 = (T)r[3 * (int64_t)v];
+        v1 = (T)r[3 * (int64_t)v + 1];
+        v2 = (T)r[3 * (int64_t)v + 2];
+    }
+    __syncthreads();
+    T s0, s1, s2;
+    restrict_sum_store_to<T>(v0, v1, v2, m, Rb, par, s0, s1, s2);
+    if(m & 0x10000)
+    {
+        const int32_t node   = par - begin1;
+        r1s[node % kBank][0] = s0;
+        r1s[node % kBank][1] = s1;
+        r1s[node % kBank][2] = s2;
+    }
+    __syncthreads();
+    if(threadIdx.x < kWave && bank1 >= 0)
+    {
+        const int     q    = threadIdx.x;
+        const int32_t node = bank1 * kBank + q;
+        const bool    in   = q < kBank && node < count1;
+        T             t0, t1, t2;
+        restrict_sum_store_to<T>(in ? r1s[q][0] : T(0), in ? r1s[q][1] : T(0), in ? r1s[q][2] : T(0),
+                                 in ? sib[begin1 + node] : 0, Rb, in ? parent[begin1 + node] : 0, t0, t1, t2);
+    }
+}
+
 // fused_update_xr (linear_fused_pcg.cu:504-549) with the level-0 restriction
 // folded in: one lane per partition slot (a whole number of workgroups),
 // then one lane per unpartitioned vertex.  A slot's lane updates x and r of
@@ -2157,6 +2213,14 @@ class MasPreconditioner final : public LocalPreconditioner
             const int32_t cnt = span.count[l];
             if(cnt == 0 || (l == 0 && r0_done) || (l == 1 && r1_done))
                 continue;
+            if(l == 0 && l1_local_ && base_lvl >= 2)
+            {
+                mas_restrict2_kernel<T><<<ceil_div(cnt, 256), 256, 0, s>>>(
+                    r, pv, R, d_parent.data(), d_sib.data(), cnt, span.begin[1], span.count[1], d_range_bank.data(),
+                    conv);
+                ++l;  // level 1 is done with it
+                continue;
+            }
             if(l == 0)
                 mas_restrict_level_kernel<T, true><<<ceil_div(cnt, 256), 256, 0, s>>>(
                     r, pv, R, d_parent.data(), d_sib.data(), span.begin[l], cnt, conv);

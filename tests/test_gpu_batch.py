@@ -232,3 +232,46 @@ def test_batch_config4_recipe(ctx):
           f"{ms:.1f} ms for the batch, iterations min {it.min()} median {int(np.median(it))} max {it.max()}",
           flush=True)
     ls.close()
+
+
+@pytest.mark.parametrize("kind", ["diag3", "mas"])
+@pytest.mark.parametrize("sizes", [[1, 341, 342, 2], [682, 683, 1, 1], [340, 1024, 17], [5]],
+                         ids=lambda s: "-".join(map(str, s)))
+def test_batch_tile_edges(ctx, sizes, kind):
+    """systems of one block row and around the tiles of 341 rows, each a chain
+    with blocks 3I on the diagonal and -I beside it: eigenvalues 1..5, so a
+    relative residual of 1e-10 leaves at most 5e-10 of error; 1e-9 for the
+    rounding of the recursion on top"""
+    seg = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    B = int(seg[-1])
+    rng = np.random.default_rng(7)
+    diag = np.arange(B, dtype=np.int32)
+    links = np.concatenate([np.arange(a, b - 1) for a, b in zip(seg[:-1], seg[1:])]).astype(np.int32)
+    rows, cols = np.concatenate([diag, links]), np.concatenate([diag, links + 1]).astype(np.int32)
+    vals = np.concatenate([np.tile(3 * np.eye(3).ravel(), (B, 1)), np.tile(-np.eye(3).ravel(), (len(links), 1))])
+    rhs = rng.standard_normal(3 * B)
+    ls = LinearSystem(ctx, B)
+    rd, cd, vd = ctx.to_device(rows), ctx.to_device(cols), ctx.to_device(vals)
+    ls.assemble(rd, cd, vd)
+    if kind == "mas":
+        # clusters of 16 vertices in a row, none across systems
+        ids, base = [], 0
+        for n in sizes:
+            ids.append(base + np.arange(n) // 16)
+            base = int(ids[-1][-1]) + 1
+        tets = np.concatenate([np.stack([np.arange(a, b - 3) + q for q in range(4)], 1) if b - a > 3 else
+                               np.zeros((0, 4), int) for a, b in zip(seg[:-1], seg[1:])])
+        ls.add_preconditioner(abi.MI_PRECOND_MAS, 0, 3 * B, part_ids=np.concatenate(ids).astype(np.int32),
+                              tets=tets.astype(np.int32))
+    else:
+        ls.add_preconditioner(abi.MI_PRECOND_DIAG3, 0, 3 * B)
+    ls.assemble_preconditioners()
+    x = ctx.alloc(3 * B, np.float64)
+    sts = ls.solve_batched(seg, ctx.to_device(rhs), x, criterion=abi.MI_CRIT_REL_RESIDUAL, tol=1e-10,
+                           max_iter_ratio=100.0)
+    xs = x.numpy().reshape(B, 3)
+    for k, n in enumerate(sizes):
+        A = 3 * np.eye(n) - np.eye(n, k=1) - np.eye(n, k=-1)
+        want = np.linalg.solve(A, rhs.reshape(B, 3)[seg[k]:seg[k + 1]])
+        assert sts[k]["converged"] == 1 and rel_err(xs[seg[k]:seg[k + 1]], want) < 1e-9, (k, n, sts[k])
+    ls.close()
