@@ -793,75 +793,97 @@ __global__ void full_count_kernel(const int32_t* lower_ptr, const int32_t* upper
     }
 }
 
-template <typename VT>
-__global__ void full_empty_kernel(const int32_t* lower_ptr,
-                                  const int32_t* upper_ptr,
-                                  const int32_t* full_ptr,
+// A layout's blocks are written in two steps: a kernel that knows the layout
+// gives every output block its index word and its source (the upper block, bit
+// 31 where it is stored transposed; kNoBlock for a zero block), and
+// fill_values_kernel moves the values.  One lane per upper block writing nine
+// planes at its own places cost more than the bytes: its stores were pieces of
+// a row's length (64^3 + 2M contacts, window layout: 276 us for the upper and 205 for
+// the lower blocks, now 48 us for words and sources and 188 for the values).
+constexpr uint32_t kTransposed = 0x80000000u;
+constexpr uint32_t kNoBlock    = 0xffffffffu;
+
+template <typename KeyT>
+__global__ void full_place_kernel(int64_t        U,
+                                  const int64_t* d_n,
+                                  const KeyT* __restrict__ keys,
+                                  KeyCodec       kc,
+                                  const int32_t* __restrict__ src,
+                                  const int32_t* __restrict__ rows,
+                                  const int32_t* __restrict__ cols,
+                                  const int32_t* __restrict__ upper_ptr,
+                                  const int32_t* __restrict__ lower_ptr,
+                                  const int32_t* __restrict__ full_ptr,
                                   int32_t        B,
-                                  int32_t*       fcols,
-                                  VT*            fvals,
-                                  int64_t        fstride)
+                                  int32_t* __restrict__ fcols,
+                                  uint32_t* __restrict__ from)
 {
-    for(int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < B; i += gridDim.x * blockDim.x)
-        if(lower_ptr[i + 1] == lower_ptr[i] && upper_ptr[i + 1] == upper_ptr[i])
-        {
-            const int64_t d = full_ptr[i];
-            fcols[d]        = i;
-#pragma unroll
-            for(int q = 0; q < 9; ++q)
-                fvals[q * fstride + d] = VT(0);
-        }
-}
-
-template <typename VT, typename KeyT>
-__global__ void full_lower_kernel(const int64_t*  d_n,
-                                  const KeyT*     keys,
-                                  KeyCodec        kc,
-                                  const int32_t*  src,
-                                  const int32_t*  lower_ptr,
-                                  const int32_t*  full_ptr,
-                                  const double*   uvals,
-                                  int32_t         B,
-                                  int32_t*        fcols,
-                                  VT*             fvals,
-                                  int64_t         fstride)
-{
+    const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
     const int64_t n = *d_n;
-    for(int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x)
-    {
-        int32_t i, j;  // lower row = upper col, lower col = upper row
-        kc.lo_rc((uint64_t)keys[k], i, j);
-        const int64_t  u   = src[k];
-        const int64_t  d   = (int64_t)full_ptr[i] + (k - lower_ptr[i]);
-        fcols[d]           = j;
-#pragma unroll
-        for(int r = 0; r < 3; ++r)
-#pragma unroll
-            for(int c = 0; c < 3; ++c)
-                fvals[(r + 3 * c) * fstride + d] = (VT)uvals[upper_at(u, c + 3 * r)];
-    }
-}
-
-template <typename VT>
-__global__ void full_upper_kernel(int64_t        U,
-                                  const int32_t* rows,
-                                  const int32_t* cols,
-                                  const int32_t* upper_ptr,
-                                  const int32_t* lower_ptr,
-                                  const int32_t* full_ptr,
-                                  const double*  uvals,
-                                  int32_t*       fcols,
-                                  VT*            fvals,
-                                  int64_t        fstride)
-{
-    for(int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < U; u += (int64_t)gridDim.x * blockDim.x)
+    for(int64_t u = t0; u < U; u += step)
     {
         const int32_t i = rows[u];
         const int64_t d = (int64_t)full_ptr[i] + (lower_ptr[i + 1] - lower_ptr[i]) + (u - upper_ptr[i]);
         fcols[d]        = cols[u];
+        from[d]         = (uint32_t)u;
+    }
+    for(int64_t k = t0; k < n; k += step)
+    {
+        int32_t i, j;  // lower row = upper col, lower col = upper row
+        kc.lo_rc((uint64_t)keys[k], i, j);
+        const int64_t d = (int64_t)full_ptr[i] + (k - lower_ptr[i]);
+        fcols[d]        = j;
+        from[d]         = (uint32_t)src[k] | kTransposed;
+    }
+    for(int64_t i = t0; i < B; i += step)
+        if(lower_ptr[i + 1] == lower_ptr[i] && upper_ptr[i + 1] == upper_ptr[i])
+        {
+            fcols[full_ptr[i]] = (int32_t)i;
+            from[full_ptr[i]]  = kNoBlock;
+        }
+}
+
+// the nine planes of *d_n blocks from their sources: memory bound.  A block's nine
+// scalars are read by nine consecutive lanes (72 B at a time, nine loads in
+// flight per lane), turned in LDS where they are stored transposed, and
+// written by plane, 256 consecutive blocks at a time.
+template <typename VT>
+__global__ __launch_bounds__(kThreads) void fill_values_kernel(const int32_t* d_n,
+                                                              const uint32_t* __restrict__ from,
+                                                              const double* __restrict__ uvals,
+                                                              VT* __restrict__ planes,
+                                                              int64_t        stride)
+{
+    __shared__ uint32_t sf[kThreads];
+    __shared__ double   sv[9 * kThreads];
+    const int64_t       n = *d_n;
+    for(int64_t d0 = (int64_t)blockIdx.x * kThreads; d0 < n; d0 += (int64_t)gridDim.x * kThreads)
+    {
+        const int nb = (int)min((int64_t)kThreads, n - d0);
+        __syncthreads();  // the last tile's blocks are read
+        if((int)threadIdx.x < nb)
+            sf[threadIdx.x] = from[d0 + threadIdx.x];
+        __syncthreads();
+        double v[9];
 #pragma unroll
-        for(int q = 0; q < 9; ++q)
-            fvals[q * fstride + d] = (VT)uvals[upper_at(u, q)];
+        for(int k = 0; k < 9; ++k)
+        {
+            const int      f = k * kThreads + threadIdx.x, j = f / 9, q = f - 9 * j;
+            const uint32_t w = j < nb ? sf[j] : kNoBlock;
+            v[k] = w == kNoBlock ? 0.0 : uvals[upper_at((int64_t)(w & ~kTransposed), q)];
+        }
+#pragma unroll
+        for(int k = 0; k < 9; ++k)
+        {
+            const int f = k * kThreads + threadIdx.x, j = f / 9, q = f - 9 * j;
+            if(j < nb)
+                sv[9 * j + ((sf[j] & kTransposed) ? 3 * (q % 3) + q / 3 : q)] = v[k];
+        }
+        __syncthreads();
+        if((int)threadIdx.x < nb)
+#pragma unroll
+            for(int q = 0; q < 9; ++q)
+                planes[q * stride + d0 + threadIdx.x] = (VT)sv[9 * threadIdx.x + q];
     }
 }
 
@@ -914,48 +936,24 @@ __host__ __device__ __forceinline__ int32_t win_inner_word(int32_t li, int32_t l
     return (int32_t)(0x80000000u | ((uint32_t)li << 15) | (uint32_t)lj);
 }
 
-template <typename VT>
-__global__ void win_upper_kernel(int64_t        U,
-                                 int            shift,
-                                 const int32_t* __restrict__ rows,
-                                 const int32_t* __restrict__ cols,
-                                 const int32_t* __restrict__ row_ptr,
-                                 const int32_t* __restrict__ pos,
-                                 const int32_t* __restrict__ wptr,
-                                 const double* __restrict__ uvals,
-                                 int32_t*       words,
-                                 VT*            wvals,
-                                 int64_t        stride)
-{
-    const int32_t mask = (1 << shift) - 1;
-    for(int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < U; u += (int64_t)gridDim.x * blockDim.x)
-    {
-        const int32_t v = rows[u], j = cols[u];
-        const int32_t p = pos[v], pj = pos[j];
-        const int64_t d = (int64_t)wptr[p] + (u - row_ptr[v]);
-        words[d]        = (p >> shift) == (pj >> shift) ? win_inner_word(p & mask, pj & mask) : pj;
-#pragma unroll
-        for(int q = 0; q < 9; ++q)
-            wvals[q * stride + d] = (VT)uvals[upper_at(u, q)];
-    }
-}
-
-template <typename VT, typename KeyT>
-__global__ __launch_bounds__(kThreads) void win_lower_kernel(int32_t        B,
+// words and sources of the window layout's blocks: 16 lanes per row, its upper
+// blocks and then the lower ones of other windows
+template <typename KeyT>
+__global__ __launch_bounds__(kThreads) void win_place_kernel(int32_t        B,
                                                             int            shift,
                                                             const int32_t* __restrict__ pos,
                                                             const int32_t* __restrict__ real,
                                                             const int32_t* __restrict__ row_ptr,
+                                                            const int32_t* __restrict__ cols,
                                                             const int32_t* __restrict__ lower_ptr,
                                                             const KeyT* __restrict__ lkeys,
                                                             KeyCodec       kc,
                                                             const int32_t* __restrict__ lsrc,
                                                             const int32_t* __restrict__ wptr,
-                                                            const double* __restrict__ uvals,
-                                                            int32_t*       words,
-                                                            VT*            wvals,
-                                                            int64_t        stride)
+                                                            int32_t* __restrict__ words,
+                                                            uint32_t* __restrict__ from)
 {
+    const int32_t mask   = (1 << shift) - 1;
     const int64_t groups = (int64_t)gridDim.x * (kThreads / kRowLanes);
     const int     lane   = threadIdx.x % kRowLanes;
     const int     gsh    = (int)(threadIdx.x % kWave) & ~(kRowLanes - 1);  // the group's first lane in the wave
@@ -970,7 +968,18 @@ __global__ __launch_bounds__(kThreads) void win_lower_kernel(int32_t        B,
         const int32_t v    = live ? real[p] : 0;
         const int32_t ch   = (int32_t)p >> shift;
         const int32_t lo = live ? lower_ptr[v] : 0, hi = live ? lower_ptr[v + 1] : 0;
-        int64_t       d  = live ? (int64_t)wptr[p] + (row_ptr[v + 1] - row_ptr[v]) : 0;
+        int64_t       d  = live ? (int64_t)wptr[p] : 0;
+        if(live)
+        {
+            const int32_t u0 = row_ptr[v], u1 = row_ptr[v + 1];
+            for(int32_t u = u0 + lane; u < u1; u += kRowLanes)
+            {
+                const int32_t pj    = pos[cols[u]];
+                words[d + (u - u0)] = (pj >> shift) == ch ? win_inner_word((int32_t)p & mask, pj & mask) : pj;
+                from[d + (u - u0)]  = (uint32_t)u;
+            }
+            d += u1 - u0;
+        }
         // the wave's longest lower list bounds its rounds
         int32_t len = hi - lo;
 #pragma unroll
@@ -993,13 +1002,8 @@ __global__ __launch_bounds__(kThreads) void win_lower_kernel(int32_t        B,
             if(out)
             {
                 const int64_t dk = d + __popc(mine & ((1u << lane) - 1u));
-                const int64_t u  = lsrc[k];
                 words[dk]        = pi;
-#pragma unroll
-                for(int r = 0; r < 3; ++r)
-#pragma unroll
-                    for(int c = 0; c < 3; ++c)
-                        wvals[(r + 3 * c) * stride + dk] = (VT)uvals[upper_at(u, c + 3 * r)];
+                from[dk]         = (uint32_t)lsrc[k] | kTransposed;
             }
             d += __popc(mine);
         }
@@ -1076,6 +1080,12 @@ void scan_exclusive(uint32_t* data, int64_t n, DBuf<uint32_t>& chunk, int64_t* t
 int grid_of(int64_t n)
 {
     return std::max(1, std::min(ceil_div(n, kThreads), device_cu_count() * 16));
+}
+
+// fill_values_kernel: its LDS allows eight workgroups per CU
+int fill_grid(int64_t n)
+{
+    return (int)std::max<int64_t>(1, std::min<int64_t>((n + kThreads - 1) / kThreads, (int64_t)device_cu_count() * 8));
 }
 }  // namespace
 
@@ -1174,44 +1184,28 @@ void MatrixConverter::build_window(BsrMatrix& A, int shape, bool want32, double 
     const int64_t wmax = 2 * U;
     A.wwords.resize((size_t)wmax + 4, ratio);
     A.wstride = ((int64_t)A.wwords.cap + 3) & ~(int64_t)3;
-    auto win_lower = [&](auto* wv) {
-        using VT = std::remove_pointer_t<decltype(wv)>;
-        if(narrow)
-            win_lower_kernel<VT, uint32_t><<<grid_of((int64_t)B * kRowLanes), kThreads, 0, s>>>(
-                B, shift, A.wpos.data(), A.wreal.data(), A.row_ptr.data(), lower_ptr_.data(),
-                key_ptr<uint32_t>(tcur_), codec(), srcs_[tcur_].data(), A.wptr.data(), A.vals.data(),
-                A.wwords.data(), wv, A.wstride);
-        else
-            win_lower_kernel<VT, uint64_t><<<grid_of((int64_t)B * kRowLanes), kThreads, 0, s>>>(
-                B, shift, A.wpos.data(), A.wreal.data(), A.row_ptr.data(), lower_ptr_.data(),
-                key_ptr<uint64_t>(tcur_), codec(), srcs_[tcur_].data(), A.wptr.data(), A.vals.data(),
-                A.wwords.data(), wv, A.wstride);
-    };
-    if(U > 0)
-    {
-        if(want32)
-        {
-            A.wvals32.resize((size_t)9 * A.wstride);
-            win_upper_kernel<float><<<grid_of(U), kThreads, 0, s>>>(U, shift, A.rows.data(), A.cols.data(),
-                                                                    A.row_ptr.data(), A.wpos.data(), A.wptr.data(),
-                                                                    A.vals.data(), A.wwords.data(), A.wvals32.data(),
-                                                                    A.wstride);
-            win_lower(A.wvals32.data());
-        }
-        else
-        {
-            A.wvals.resize((size_t)9 * A.wstride);
-            win_upper_kernel<double><<<grid_of(U), kThreads, 0, s>>>(U, shift, A.rows.data(), A.cols.data(),
-                                                                     A.row_ptr.data(), A.wpos.data(), A.wptr.data(),
-                                                                     A.vals.data(), A.wwords.data(), A.wvals.data(),
-                                                                     A.wstride);
-            win_lower(A.wvals.data());
-        }
-    }
-    else if(want32)
+    if(want32)
         A.wvals32.resize((size_t)9 * A.wstride);
     else
         A.wvals.resize((size_t)9 * A.wstride);
+    if(U > 0)
+    {
+        from_.resize((size_t)wmax, ratio);
+        if(narrow)
+            win_place_kernel<uint32_t><<<grid_of((int64_t)B * kRowLanes), kThreads, 0, s>>>(
+                B, shift, A.wpos.data(), A.wreal.data(), A.row_ptr.data(), A.cols.data(), lower_ptr_.data(),
+                key_ptr<uint32_t>(tcur_), codec(), srcs_[tcur_].data(), A.wptr.data(), A.wwords.data(), from_.data());
+        else
+            win_place_kernel<uint64_t><<<grid_of((int64_t)B * kRowLanes), kThreads, 0, s>>>(
+                B, shift, A.wpos.data(), A.wreal.data(), A.row_ptr.data(), A.cols.data(), lower_ptr_.data(),
+                key_ptr<uint64_t>(tcur_), codec(), srcs_[tcur_].data(), A.wptr.data(), A.wwords.data(), from_.data());
+        if(want32)
+            fill_values_kernel<float><<<fill_grid(wmax), kThreads, 0, s>>>(A.wptr.data() + B, from_.data(),
+                                                                           A.vals.data(), A.wvals32.data(), A.wstride);
+        else
+            fill_values_kernel<double><<<fill_grid(wmax), kThreads, 0, s>>>(A.wptr.data() + B, from_.data(),
+                                                                            A.vals.data(), A.wvals.data(), A.wstride);
+    }
     MI_HIP(hipGetLastError());
     A.wblocks = -1;  // read back lazily (window_blocks)
     A.has_win = true;
@@ -1461,40 +1455,26 @@ void MatrixConverter::build_full(BsrMatrix& out, bool want32, double ratio, hipS
     // an even plane stride keeps every pair 8-byte aligned
     out.fcols.resize((size_t)fmax + 2, ratio);
     out.fstride = ((int64_t)out.fcols.cap + 1) & ~(int64_t)1;
-    auto full_lower = [&](auto* fv) {
-        using VT = std::remove_pointer_t<decltype(fv)>;
-        if(narrow)
-            full_lower_kernel<VT, uint32_t><<<grid_of(U), kThreads, 0, s>>>(
-                d_off, key_ptr<uint32_t>(tcur), codec(), srcs_[tcur].data(), lower_ptr_.data(), out.full_ptr.data(),
-                out.vals.data(), B, out.fcols.data(), fv, out.fstride);
-        else
-            full_lower_kernel<VT, uint64_t><<<grid_of(U), kThreads, 0, s>>>(
-                d_off, key_ptr<uint64_t>(tcur), codec(), srcs_[tcur].data(), lower_ptr_.data(), out.full_ptr.data(),
-                out.vals.data(), B, out.fcols.data(), fv, out.fstride);
-    };
+    from_.resize((size_t)fmax, ratio);
+    if(narrow)
+        full_place_kernel<uint32_t><<<grid_of(std::max(U, (int64_t)B)), kThreads, 0, s>>>(
+            U, d_off, key_ptr<uint32_t>(tcur), codec(), srcs_[tcur].data(), out.rows.data(), out.cols.data(),
+            out.row_ptr.data(), lower_ptr_.data(), out.full_ptr.data(), B, out.fcols.data(), from_.data());
+    else
+        full_place_kernel<uint64_t><<<grid_of(std::max(U, (int64_t)B)), kThreads, 0, s>>>(
+            U, d_off, key_ptr<uint64_t>(tcur), codec(), srcs_[tcur].data(), out.rows.data(), out.cols.data(),
+            out.row_ptr.data(), lower_ptr_.data(), out.full_ptr.data(), B, out.fcols.data(), from_.data());
     if(want32)
     {
         out.fvals32.resize((size_t)9 * out.fstride);
-        full_lower(out.fvals32.data());
-        full_upper_kernel<float><<<grid_of(U), kThreads, 0, s>>>(U, out.rows.data(), out.cols.data(),
-                                                                 out.row_ptr.data(), lower_ptr_.data(),
-                                                                 out.full_ptr.data(), out.vals.data(),
-                                                                 out.fcols.data(), out.fvals32.data(), out.fstride);
-        full_empty_kernel<float><<<grid_of(B), kThreads, 0, s>>>(lower_ptr_.data(), out.row_ptr.data(),
-                                                                 out.full_ptr.data(), B, out.fcols.data(),
-                                                                 out.fvals32.data(), out.fstride);
+        fill_values_kernel<float><<<fill_grid(fmax), kThreads, 0, s>>>(out.full_ptr.data() + B, from_.data(),
+                                                                       out.vals.data(), out.fvals32.data(), out.fstride);
     }
     else
     {
         out.fvals.resize((size_t)9 * out.fstride);
-        full_lower(out.fvals.data());
-        full_upper_kernel<double><<<grid_of(U), kThreads, 0, s>>>(U, out.rows.data(), out.cols.data(),
-                                                                  out.row_ptr.data(), lower_ptr_.data(),
-                                                                  out.full_ptr.data(), out.vals.data(),
-                                                                  out.fcols.data(), out.fvals.data(), out.fstride);
-        full_empty_kernel<double><<<grid_of(B), kThreads, 0, s>>>(lower_ptr_.data(), out.row_ptr.data(),
-                                                                  out.full_ptr.data(), B, out.fcols.data(),
-                                                                  out.fvals.data(), out.fstride);
+        fill_values_kernel<double><<<fill_grid(fmax), kThreads, 0, s>>>(out.full_ptr.data() + B, from_.data(),
+                                                                        out.vals.data(), out.fvals.data(), out.fstride);
     }
     out.has_full = true;
     MI_HIP(hipGetLastError());

@@ -190,6 +190,7 @@ class MatrixConverter
     DBuf<int32_t>  srcs_[2];
     DBuf<uint32_t> hist_, chunk_;
     DBuf<uint32_t> tile_cnt_;
+    DBuf<uint32_t> from_;      // the source of every block of a layout being built
     DBuf<uint32_t> seg_tile_;  // unique blocks before every tile of the segmented reduce
     DBuf<int32_t>  seg_start_, lower_ptr_;
     DBuf<int64_t>  counts_;  // [0] kept triplets, [1] U, [2] off-diagonal upper blocks, [3] full, [4] window blocks

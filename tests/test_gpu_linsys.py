@@ -323,6 +323,40 @@ def test_spmv_layout_by_size(ctx, precision, grid, rows):
     ls.close()
 
 
+@pytest.mark.parametrize("precision", [abi.MI_FP64, abi.MI_FP32])
+@pytest.mark.parametrize("shape", [abi.MI_SPMV_SHAPE_FULL, 0, 12])
+@pytest.mark.parametrize("B,links", [(1, 0), (3, 0), (40, 88), (40, 89), (200, 300), (530, 2400)])
+def test_layout_blocks_from_sources(ctx, B, links, shape, precision):
+    """unsymmetric blocks on `links` off-diagonal places and the diagonal of every
+    second row (the other rows may be empty), so that the layouts hold one block,
+    around one and several tiles of 256, zero blocks and transposed ones; the
+    product against numpy's, to the rounding of a sum of at most 3B terms"""
+    rng = np.random.default_rng(B + links)
+    iu, ju = np.triu_indices(B, 1)
+    pick = rng.permutation(len(iu))[:links]
+    diag = np.arange(0, B, 2)
+    rows = np.concatenate([diag, iu[pick]]).astype(np.int32)
+    cols = np.concatenate([diag, ju[pick]]).astype(np.int32)
+    vals = rng.standard_normal((len(rows), 3, 3))
+    vals[:len(diag)] += np.swapaxes(vals[:len(diag)], 1, 2)
+    A = np.zeros((B, 3, B, 3))
+    for i, j, v in zip(rows, cols, vals):
+        A[i, :, j] = v.T  # triplet values are column-major
+        A[j, :, i] = v
+    A = A.reshape(3 * B, 3 * B)
+    x = rng.standard_normal(3 * B)
+    ls = LinearSystem(ctx, B, precision)
+    ls.set_spmv_shape(shape)
+    rd, cd, vd = ctx.to_device(rows), ctx.to_device(cols), ctx.to_device(vals.reshape(-1, 9))
+    ls.assemble(rd, cd, vd)
+    y = ctx.alloc(3 * B, np.float64)
+    ls.spmv_dot(ctx.to_device(x), y)
+    eps = np.finfo(np.float64 if precision == abi.MI_FP64 else np.float32).eps
+    bound = (3 * B + 2) * eps * (np.abs(A) @ np.abs(x)).max()
+    assert np.abs(y.numpy() - A @ x).max() <= bound
+    ls.close()
+
+
 def test_pcg_after_a_shape_change(ctx, c1_contact):
     """a solve captured in a HIP graph with one SpMV layout is not replayed
     after the layout changes (another window size, the full BSR, the size's
