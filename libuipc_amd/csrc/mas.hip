@@ -923,11 +923,12 @@ __global__ __launch_bounds__(64) void mas_invert_kernel(const double* __restrict
 }
 
 // The same inverse on FP64 matrix cores: one wave per cluster, the 48x48
-// matrix resident in MFMA accumulators (3x3 tiles of 16x16; tile (I, J)
-// entry v of lane 16g + c holds S(16I + 4v + g, 16J + c)), swept in twelve
+// matrix's tiles on and above the diagonal resident in MFMA accumulators (six of
+// 16x16; tile (I, J), J >= I, entry v of lane 16g + c holds
+// S(16I + 4v + g, 16J + c)), swept in twelve
 // pivot panels of 4 rows.  For panel K, with P = S_KK = L L^T (Cholesky):
 //   W   = L^-1 S_K,:  (its K columns zero)
-//   S  -= W^T W                    nine v_mfma_f64_16x16x4, one per tile
+//   S  -= W^T W                    six v_mfma_f64_16x16x4, one per tile
 //   S_K,: = L^-T W,  S_:,K = its transpose,  S_KK = -L^-T L^-1
 // which is the symmetric sweep S_ij -= S_iK P^-1 S_Kj, S_Kj <- P^-1 S_Kj,
 // S_KK <- -P^-1 with the Schur update in its Cholesky form: the explicit
@@ -939,30 +940,44 @@ __global__ __launch_bounds__(64) void mas_invert_kernel(const double* __restrict
 // 36 addresses per lane).  Both MFMA operands of tile (I, J) are lane values of W
 // (A = W_I^T: lane 16g + c holds W(g, 16I + c); B = W_J: W(g, 16J + c)), so
 // a lane computes three values of W per panel; the panel's rows, W and
-// L^-T W pass between lanes through 4.5 KB of LDS.  The 4x4 Cholesky
+// L^-T W pass between lanes through the same LDS.  The 4x4 Cholesky
 // factor and its inverse run redundantly on every lane.  No pivoting, as in
 // the reference's sweep: the cluster matrices are SPD and a zero diagonal (a
 // padding slot) is set to 1.
+//
+// Bound by its instructions (about 3,900 per cluster, of them 960 FP64 and 72
+// MFMA; nine tiles with selects that had become branches took 7,000): 41^3 vertices
+// 109 -> 85 us.  Three waves per SIMD (168 registers, 30 spilled) 94 us.
 //
 // v_mfma_f64_16x16x4 lane layout (lane l, g = l / 16, c = l % 16):
 //   A operand A[c][g], B operand B[g][c], accumulator v holds D[4 v + g][c]
 // (checked on gfx950 with distinct, unsymmetric operands).
 typedef double mfma_f64x4 __attribute__((ext_vector_type(4)));
 
+// one of four by the low bits of q: selects (a chain of comparisons with q becomes
+// a switch, and its cases branches)
+__device__ __forceinline__ double select4(int q, double a, double b, double c, double d)
+{
+    const double lo = (q & 1) ? b : a, hi = (q & 1) ? d : c;
+    return (q & 2) ? hi : lo;
+}
+
 template <typename TO>
 __global__ __launch_bounds__(64, 2) void mas_invert_mfma_kernel(const double* __restrict__ hess, TO* inv, int64_t C)
 {
     constexpr int D = 3 * kBank;
-    __shared__ double Ms[kCm];     // the cluster's upper blocks in, its inverse's planes out
-    __shared__ double rowb[4][D];  // the panel's rows of S
-    __shared__ double wb[4][D];    // W
-    __shared__ double xb[4][D];    // L^-T W
+    __shared__ double Ms[kCm];  // the cluster's upper blocks in, its inverse's planes out
+    // between the two, in the same place:
+    double(*rowb)[D] = reinterpret_cast<double(*)[D]>(Ms);           // the panel's rows of S
+    double(*wb)[D]   = reinterpret_cast<double(*)[D]>(Ms + 4 * D);   // W
+    double(*xb)[D]   = reinterpret_cast<double(*)[D]>(Ms + 8 * D);   // L^-T W
+    static_assert(12 * D <= kCm, "the panels fit the cluster's copy");
     const int         lane = threadIdx.x;
     const int         g = lane >> 4, c = lane & 15;
     const int64_t     k = blockIdx.x;
     const double*     M = hess + k * kCm;
     // the upper blocks (9 column-major scalars each), staged by coalesced
-    // loads, into both triangles
+    // loads, into the tiles on and above the diagonal
     for(int e = lane; e < kCm; e += kWave)
         Ms[e] = M[e];
     __syncthreads();
@@ -970,17 +985,21 @@ __global__ __launch_bounds__(64, 2) void mas_invert_mfma_kernel(const double* __
 #pragma unroll
     for(int I = 0; I < 3; ++I)
 #pragma unroll
-        for(int J = 0; J < 3; ++J)
+        for(int J = I; J < 3; ++J)
 #pragma unroll
             for(int v = 0; v < 4; ++v)
             {
                 const int row = 16 * I + 4 * v + g, col = 16 * J + c;
                 const int a = row / 3, ra = row % 3, b = col / 3, cb = col % 3;
-                double val = a <= b ? Ms[9 * sym_index(a, b) + ra + 3 * cb] : Ms[9 * sym_index(b, a) + cb + 3 * ra];
-                if(row == col && val == 0.0)
-                    val = 1.0;
-                S[I][J][v] = val;
+                // (below a diagonal tile's diagonal blocks, the transposed entry;
+                // one address either way: two loads under a branch each way
+                // and the stores' branches below were a third of the kernel's
+                // instructions)
+                const bool   up  = I != J || a <= b;
+                const double val = Ms[9 * sym_index(up ? a : b, up ? b : a) + (up ? ra + 3 * cb : cb + 3 * ra)];
+                S[I][J][v]       = I == J && row == col && val == 0.0 ? 1.0 : val;
             }
+    __syncthreads();  // Ms is read
 #pragma unroll
     for(int J = 0; J < 3; ++J)
         rowb[g][16 * J + c] = S[0][J][0];
@@ -1026,15 +1045,25 @@ __global__ __launch_bounds__(64, 2) void mas_invert_mfma_kernel(const double* __
             }
         }
         // the lane's row and column of L^-1 (g is a lane value: selects, not
-        // an indexed array, keep Li in registers)
+        // an indexed array, keep Li in registers); the empty asm keeps the
+        // compiler from moving their computation into branches for each g
+#pragma unroll
+        for(int m = 0; m < 4; ++m)
+#pragma unroll
+            for(int n = 0; n <= m; ++n)
+                asm("" : "+v"(Li[m][n]));
         double lrow[4], lcol[4];
 #pragma unroll
         for(int m = 0; m < 4; ++m)
         {
-            lrow[m] = g == 0 ? Li[0][m] : g == 1 ? Li[1][m] : g == 2 ? Li[2][m] : Li[3][m];
-            lcol[m] = g == 0 ? Li[m][0] : g == 1 ? Li[m][1] : g == 2 ? Li[m][2] : Li[m][3];
+            lrow[m] = select4(g, Li[0][m], Li[1][m], Li[2][m], Li[3][m]);
+            lcol[m] = select4(g, Li[m][0], Li[m][1], Li[m][2], Li[m][3]);
         }
-        // W(g, 16T + c) = sum_m Li[g][m] S(k0 + m, 16T + c), zero in the K columns
+        const int  mk  = c - ko;  // the lane's column in the panel
+        const bool inK = mk >= 0 && mk < 4;
+        const double lk = select4(mk, lrow[0], lrow[1], lrow[2], lrow[3]);
+        // W(g, 16T + c) = sum_m Li[g][m] S(k0 + m, 16T + c), zero in the K columns;
+        // X takes L^-1 there, which gives L^-T L^-1
         double w[3];
 #pragma unroll
         for(int T = 0; T < 3; ++T)
@@ -1043,11 +1072,11 @@ __global__ __launch_bounds__(64, 2) void mas_invert_mfma_kernel(const double* __
 #pragma unroll
             for(int m = 0; m < 4; ++m)
                 t += lrow[m] * rowb[m][16 * T + c];
-            w[T]             = (T == Kt && c >= ko && c < ko + 4) ? 0.0 : t;
-            wb[g][16 * T + c] = w[T];
+            w[T]              = T == Kt && inK ? 0.0 : t;
+            wb[g][16 * T + c] = T == Kt && inK ? lk : t;
         }
         __syncthreads();
-        // X(g, 16T + c) = sum_{q >= g} Li[q][g] W(q, 16T + c)
+        // X(g, 16T + c) = sum_{q >= g} Li[q][g] W(q, 16T + c), negative in the pivot block
         double x[3];
 #pragma unroll
         for(int T = 0; T < 3; ++T)
@@ -1056,41 +1085,50 @@ __global__ __launch_bounds__(64, 2) void mas_invert_mfma_kernel(const double* __
 #pragma unroll
             for(int q = 0; q < 4; ++q)
                 t += lcol[q] * wb[q][16 * T + c];
-            x[T]             = t;
-            xb[g][16 * T + c] = t;
+            x[T]              = T == Kt && inK ? -t : t;
+            xb[g][16 * T + c] = x[T];
         }
         // S -= W^T W
 #pragma unroll
         for(int I = 0; I < 3; ++I)
 #pragma unroll
-            for(int J = 0; J < 3; ++J)
+            for(int J = I; J < 3; ++J)
                 S[I][J] = __builtin_amdgcn_mfma_f64_16x16x4f64(-w[I], w[J], S[I][J], 0, 0, 0);
         __syncthreads();
-        // the pivot rows (lane row k0 + g), then the pivot columns (lanes of
-        // columns k0 .. k0 + 3), then the pivot block
+        // the pivot columns (lanes of columns k0 .. k0 + 3), then the pivot rows
+        // (lane row k0 + g) with the pivot block
+        // (the loads are every lane's and stay before the selects, as above)
+        double t[3][4];
 #pragma unroll
-        for(int J = 0; J < 3; ++J)
+        for(int I = 0; I <= Kt; ++I)
+#pragma unroll
+            for(int v = 0; v < 4; ++v)
+                t[I][v] = xb[mk & 3][16 * I + 4 * v + g];
+#pragma unroll
+        for(int I = 0; I <= Kt; ++I)
+#pragma unroll
+            for(int v = 0; v < 4; ++v)
+            {
+                asm("" : "+v"(t[I][v]));
+                S[I][Kt][v] = inK ? t[I][v] : S[I][Kt][v];
+            }
+#pragma unroll
+        for(int J = Kt; J < 3; ++J)
             S[Kt][J][vK] = x[J];
-        if(c >= ko && c < ko + 4)
-        {
-            const int m = c - ko;
-#pragma unroll
-            for(int I = 0; I < 3; ++I)
-#pragma unroll
-                for(int v = 0; v < 4; ++v)
-                    S[I][Kt][v] = xb[m][16 * I + 4 * v + g];
-            double t = 0.0;
-#pragma unroll
-            for(int q = 0; q < 4; ++q)
-                t += lcol[q] * (m == 0 ? Li[q][0] : m == 1 ? Li[q][1] : m == 2 ? Li[q][2] : Li[q][3]);
-            S[Kt][Kt][vK] = -t;
-        }
         if(kp + 1 < D / 4)
         {
-            const int k1 = k0 + 4, Kt1 = k1 / 16, vK1 = (k1 % 16) / 4;
+            // the next panel's rows: along the tiles right of the diagonal, and
+            // as the columns of those above it
+            const int k1 = k0 + 4, Kt1 = k1 / 16, ko1 = k1 % 16, vK1 = ko1 / 4;
 #pragma unroll
-            for(int J = 0; J < 3; ++J)
+            for(int J = Kt1; J < 3; ++J)
                 rowb[g][16 * J + c] = S[Kt1][J][vK1];
+            if(c >= ko1 && c < ko1 + 4 && Kt1 > 0)
+#pragma unroll
+                for(int J = 0; J < Kt1; ++J)
+#pragma unroll
+                    for(int v = 0; v < 4; ++v)
+                        rowb[c - ko1][16 * J + 4 * v + g] = S[J][Kt1][v];
         }
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);  // no work moves between panels (register pressure)
@@ -1101,22 +1139,20 @@ __global__ __launch_bounds__(64, 2) void mas_invert_mfma_kernel(const double* __
 #pragma unroll
     for(int I = 0; I < 3; ++I)
 #pragma unroll
-        for(int J = 0; J < 3; ++J)
+        for(int J = I; J < 3; ++J)
 #pragma unroll
             for(int v = 0; v < 4; ++v)
             {
                 const int    row = 16 * I + 4 * v + g, col = 16 * J + c;
                 const int    a = row / 3, ra = row % 3, b = col / 3, cb = col % 3;
                 const double val = -S[I][J][v];
-                if(a < b)
-                    Ms[inv_at(sym_index(a, b), ra + 3 * cb)] = val;
-                else if(a == b && ra <= cb)
-                {
-                    const int si = sym_index(a, a);
+                const int    si  = sym_index(a, b);
+                // right of the diagonal tiles every entry is above the diagonal, and only
+                // the last four rows share a block with the next tile's columns
+                if(I != J || row <= col)
                     Ms[inv_at(si, ra + 3 * cb)] = val;
-                    if(ra < cb)
-                        Ms[inv_at(si, cb + 3 * ra)] = val;
-                }
+                if((I == J || (J == I + 1 && v == 3)) && a == b && row < col)
+                    Ms[inv_at(si, cb + 3 * ra)] = val;
             }
     __syncthreads();
     TO* O = inv + k * kCm;
