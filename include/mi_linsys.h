@@ -473,7 +473,10 @@ typedef struct mi_pcg_opts
     double  tol;            /* reference default tol_rate = 1e-3 (scene_default_config.cpp:146) */
     double  max_iter_ratio; /* max_iter = ratio * n (reference: 2)                         */
     int32_t check_interval; /* iterations between convergence checks (reference: 5)        */
-    int32_t use_graph;      /* 1: replay a captured hipGraph of graph_checks check intervals */
+    int32_t use_graph;      /* 1: replay a captured hipGraph of graph_checks check intervals, or, up to
+                             * 16,384 block rows on the full BSR in the caller's vector order with
+                             * one DIAG3 or whole-vector MAS or no preconditioner, run the iterations
+                             * in one cooperative launch (env MI_PCG_SMALL=0: always the graph) */
     int32_t psd_fallback;   /* 1: rz0 < 0 or non-finite -> plain CG (linear_fused_pcg.cu:1843-1875) */
     int32_t force_bypass;   /* 1: always bypass the preconditioner (UIPC_PCG_PSD_FALLBACK_TEST) */
     int32_t true_residual;  /* 1: compute ||b - A x|| / ||b|| after the solve (one SpMV)    */

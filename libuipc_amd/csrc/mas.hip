@@ -20,14 +20,16 @@
 //            entry has exactly one source, so a plain store), then up the levels
 //            adding the block where its two ancestors are different nodes of one
 //            bank (FP64 atomics, wave-aggregated when few destinations repeat);
-//            the walk stops where the ancestors merge;
+//            the walk stops where the ancestors merge; where every level-1 bank is
+//            a 256-slot range, a workgroup per range sums its coarse clusters in
+//            LDS and does their pushes too;
 //     push   level by level, the full sum of every group of nodes that share a
 //            parent becomes the parent's diagonal block (plain store; a parent's
 //            children all live in one bank).  This replaces the reference's
 //            per-block diagonal atomics at every level above the merge, which
 //            would all land on the few top-level blocks.
-//   invert one wave per cluster, FP64 symmetric Gauss-Jordan sweep
-//          (the sweep of 1077-1175, in double); zero diagonal -> 1; stored as
+//   invert one wave per cluster, FP64 symmetric sweep on matrix cores, or the
+//          column sweep of 1077-1175 in double; zero diagonal -> 1; stored as
 //          FP64 or FP32 upper blocks.
 //
 // Apply (per PCG iteration, GPU; 2887-2960):
