@@ -333,6 +333,9 @@ __device__ __forceinline__ uint64_t lanemask_lt64()
 // of its contiguous quarter of the tile in order (ballot-matched peers +
 // per-wave digit counters), the tile is reordered by digit in LDS, then each
 // digit run is written out contiguously.
+// (Counting by returning LDS atomics, so that no round waits for the one
+// before: 142 -> 160 us per pass of the 64^3 + 2M system; the other waves hide
+// that chain.)
 // totals: the digits' totals (many tiles).
 template <typename KeyT, typename Src, bool kFew>
 __global__ __launch_bounds__(kThreads) void rs_scatter_kernel(Src             src,
