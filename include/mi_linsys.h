@@ -476,7 +476,8 @@ typedef struct mi_pcg_opts
     int32_t use_graph;      /* 1: replay a captured hipGraph of graph_checks check intervals, or, up to
                              * 16,384 block rows on the full BSR in the caller's vector order with
                              * one DIAG3 or whole-vector MAS or no preconditioner, run the iterations
-                             * in one cooperative launch (env MI_PCG_SMALL=0: always the graph) */
+                             * in one cooperative launch (mi_sys_set_one_launch; env MI_PCG_SMALL=0:
+                             * always the graph) */
     int32_t psd_fallback;   /* 1: rz0 < 0 or non-finite -> plain CG (linear_fused_pcg.cu:1843-1875) */
     int32_t force_bypass;   /* 1: always bypass the preconditioner (UIPC_PCG_PSD_FALLBACK_TEST) */
     int32_t true_residual;  /* 1: compute ||b - A x|| / ||b|| after the solve (one SpMV)    */
@@ -520,6 +521,15 @@ int mi_pcg_solve(mi_sys*            sys,
                  const mi_pcg_opts* opts,
                  mi_pcg_stats*      stats_host,
                  void*              stream);
+
+/* The one-launch iterations of mi_pcg_solve on small systems (mi_pcg_opts.use_graph;
+ * no counterpart in the reference).  A cooperative launch runs up to 512
+ * iterations.  mi_sys_set_one_launch: the most launches a solve of this system
+ * uses before it goes on with the captured graph; -1 (the default): no limit,
+ * 0: the graph from the start.  mi_sys_one_launch: how many the last solve used
+ * (0: it ran on the graph or on plain launches). */
+int mi_sys_set_one_launch(mi_sys* sys, int32_t max_launches);
+int mi_sys_one_launch(mi_sys* sys, int32_t* launches);
 
 /* Batched PCG: the system holds nseg independent systems on the block-row
  * ranges [seg_rows_host[k], seg_rows_host[k + 1]) (seg_rows_host[0] = 0,

@@ -104,8 +104,10 @@ struct mi_sys
     } graph_key;
     bool graph_failed = false;
 
-    // small systems: the iterations in one cooperative launch
+    // small systems: the iterations in one cooperative launch (mi_sys_set_one_launch)
     SmallPcgScratch small;
+    int32_t         one_launch_max  = -1;  // launches a solve may use (-1: no limit)
+    int32_t         one_launch_done = 0;   // launches of the last solve
 
     // batched solves (mi_pcg_solve_batched): the tile table of the last
     // segmentation, per-system scalars, tile partials and their own graph
@@ -723,6 +725,23 @@ int mi_sys_set_spmv_shape(mi_sys* sys, int32_t shape, void* stream)
     const int want = layout_shape(sys);
     if(sys->assembled && (want < 0 ? sys->A.has_win : (!sys->A.has_win || sys->A.wshape != want)))
         build_spmv_layout(sys, pick(sys->ctx, stream));
+    MI_API_END
+}
+
+int mi_sys_set_one_launch(mi_sys* sys, int32_t max_launches)
+{
+    MI_API_BEGIN
+    MI_REQUIRE(sys, MI_ERR_ARG, "mi_sys_set_one_launch: null sys");
+    MI_REQUIRE(max_launches >= -1, MI_ERR_ARG, "mi_sys_set_one_launch: max_launches must be -1 or more");
+    sys->one_launch_max = max_launches;
+    MI_API_END
+}
+
+int mi_sys_one_launch(mi_sys* sys, int32_t* launches)
+{
+    MI_API_BEGIN
+    MI_REQUIRE(sys && launches, MI_ERR_ARG, "mi_sys_one_launch: null argument");
+    *launches = sys->one_launch_done;
     MI_API_END
 }
 
@@ -1444,6 +1463,7 @@ extern "C" int mi_pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pc
     const int64_t n = sys->n();
     *st             = mi_pcg_stats{};
     st->rel_res_true = NAN;
+    sys->one_launch_done = 0;
     if(n == 0)
     {
         st->converged = 1;
@@ -1626,10 +1646,11 @@ extern "C" int mi_pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pc
                 one_launch = sys->pcs.size() == 1 && sys->pcs[0]->small_pcg(sm);
         }
     }
-    while(one_launch && done < total)
+    while(one_launch && done < total && (sys->one_launch_max < 0 || sys->one_launch_done < sys->one_launch_max))
     {
         if(!pcg_small_launch(sm, sys->small, total - done, s))
             break;
+        ++sys->one_launch_done;
         read_scalars(sys, s);
         MI_REQUIRE(!h.stalled, MI_ERR_HIP, "mi_pcg_solve: a wait between workgroups ran out");
         MI_REQUIRE(std::isfinite(h.rz_new), MI_ERR_NONFINITE,
@@ -1643,6 +1664,9 @@ extern "C" int mi_pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pc
             break;
         }
     }
+    // the one-launch iterations leave p in double only
+    if(!converged && sys->one_launch_done > 0 && use32_sys && !sys->A.has_win)
+        pack_f32x4(sys->p.data(), sys->p32.data(), sys->desc.block_rows, s);
     while(!converged && done < total)
     {
         int64_t blk       = std::min<int64_t>(gb, total - done);

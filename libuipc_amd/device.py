@@ -247,6 +247,16 @@ class LinearSystem:
         """the window kernel's launch shape (an assembled layout is rebuilt)"""
         check(self.lib.mi_sys_set_spmv_shape(self.h, int(shape), stream))
 
+    def set_one_launch(self, max_launches: int) -> None:
+        """the most cooperative launches a solve uses (-1: no limit, 0: the graph)"""
+        check(self.lib.mi_sys_set_one_launch(self.h, int(max_launches)))
+
+    def one_launch(self) -> int:
+        """the cooperative launches of the last solve"""
+        n = C.c_int32()
+        check(self.lib.mi_sys_one_launch(self.h, C.byref(n)))
+        return n.value
+
     def spmv_layout(self) -> dict:
         """the layout the SpMV streams: window (1) or full BSR (0), window rows,
         workgroup size and blocks per product"""
