@@ -527,8 +527,14 @@ int mi_pcg_solve(mi_sys*            sys,
  * iterations.  mi_sys_set_one_launch: the most launches a solve of this system
  * uses before it goes on with the captured graph; -1 (the default): no limit,
  * 0: the graph from the start.  mi_sys_one_launch: how many the last solve used
- * (0: it ran on the graph or on plain launches). */
+ * (0: it ran on the graph or on plain launches).
+ * The launch's workgroups wait for each other.  Where a wait runs out (they do not
+ * all run, as when another process holds a part of the GPU in the same way), the
+ * solve starts again on the graph, and the system stays on it until one of the
+ * two setters is called.  mi_sys_set_one_launch_wait: how long a wait lasts, in
+ * microseconds; -1 (the default): 4 s; 0: it ends at its first look. */
 int mi_sys_set_one_launch(mi_sys* sys, int32_t max_launches);
+int mi_sys_set_one_launch_wait(mi_sys* sys, int64_t microseconds);
 int mi_sys_one_launch(mi_sys* sys, int32_t* launches);
 
 /* Batched PCG: the system holds nseg independent systems on the block-row

@@ -168,6 +168,7 @@ LINSYS_PROTOS = {
     "mi_spmv_shapes": (C.c_int, [C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.c_void_p, C.c_void_p, C.c_void_p,
                                  C.c_void_p]),
     "mi_sys_set_one_launch": (C.c_int, [C.c_void_p, C.c_int32]),
+    "mi_sys_set_one_launch_wait": (C.c_int, [C.c_void_p, C.c_int64]),
     "mi_sys_one_launch": (C.c_int, [C.c_void_p, C.POINTER(C.c_int32)]),
     "mi_sys_set_spmv_shape": (C.c_int, [C.c_void_p, C.c_int32, C.c_void_p]),
     "mi_sys_spmv_layout": (C.c_int, [C.c_void_p, C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.POINTER(C.c_int32),

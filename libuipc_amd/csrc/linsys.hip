@@ -107,7 +107,9 @@ struct mi_sys
     // small systems: the iterations in one cooperative launch (mi_sys_set_one_launch)
     SmallPcgScratch small;
     int32_t         one_launch_max  = -1;  // launches a solve may use (-1: no limit)
+    int64_t         one_launch_wait = -1;  // ticks that a workgroup waits (-1: the default)
     int32_t         one_launch_done = 0;   // launches of the last solve
+    bool            one_launch_off  = false;  // a wait ran out: the graph from then on
 
     // batched solves (mi_pcg_solve_batched): the tile table of the last
     // segmentation, per-system scalars, tile partials and their own graph
@@ -734,6 +736,18 @@ int mi_sys_set_one_launch(mi_sys* sys, int32_t max_launches)
     MI_REQUIRE(sys, MI_ERR_ARG, "mi_sys_set_one_launch: null sys");
     MI_REQUIRE(max_launches >= -1, MI_ERR_ARG, "mi_sys_set_one_launch: max_launches must be -1 or more");
     sys->one_launch_max = max_launches;
+    sys->one_launch_off = false;
+    MI_API_END
+}
+
+int mi_sys_set_one_launch_wait(mi_sys* sys, int64_t microseconds)
+{
+    MI_API_BEGIN
+    MI_REQUIRE(sys, MI_ERR_ARG, "mi_sys_set_one_launch_wait: null sys");
+    MI_REQUIRE(microseconds >= -1 && microseconds <= 60000000, MI_ERR_ARG,
+               "mi_sys_set_one_launch_wait: -1 or 0 to 60,000,000 microseconds");
+    sys->one_launch_wait = microseconds < 0 ? -1 : 100 * microseconds;
+    sys->one_launch_off  = false;
     MI_API_END
 }
 
@@ -1444,30 +1458,19 @@ struct RowOrderScope
             pc->set_row_order(false);
     }
 };
-}  // namespace
 
-extern "C" int mi_pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pcg_opts* opts, mi_pcg_stats* st, void* stream)
+// one solve; false: a wait between the workgroups of a cooperative launch ran out
+// (x, the vectors and st are then undefined, x0 is in sys->small.x0 if one was given)
+bool pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pcg_opts& o, mi_pcg_stats* st, hipStream_t s)
 {
-    MI_API_BEGIN
-    MI_REQUIRE(sys && b && x && st, MI_ERR_ARG, "mi_pcg_solve: null argument");
-    MI_REQUIRE(sys->assembled, MI_ERR_STATE, "mi_pcg_solve: system not assembled");
-    MI_REQUIRE(sys->pcs.empty() || sys->pcs_assembled, MI_ERR_STATE, "mi_pcg_solve: preconditioners not assembled");
-    mi_pcg_opts o;
-    mi_pcg_default_opts(&o);
-    if(opts)
-        o = *opts;
-    MI_REQUIRE(o.tol > 0.0 && o.max_iter_ratio > 0.0, MI_ERR_ARG, "mi_pcg_solve: tol and max_iter_ratio must be > 0");
-    MI_REQUIRE(o.criterion == MI_CRIT_RZ_RATIO || o.criterion == MI_CRIT_REL_RESIDUAL, MI_ERR_ARG,
-               "mi_pcg_solve: unknown criterion");
-    hipStream_t   s = pick(sys->ctx, stream);
-    const int64_t n = sys->n();
-    *st             = mi_pcg_stats{};
+    const int64_t n  = sys->n();
+    *st              = mi_pcg_stats{};
     st->rel_res_true = NAN;
     sys->one_launch_done = 0;
     if(n == 0)
     {
         st->converged = 1;
-        return MI_OK;
+        return true;
     }
     double ratio = sys->desc.reserve_ratio;
     sys->r.resize((size_t)n, ratio);
@@ -1580,7 +1583,7 @@ extern "C" int mi_pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pc
         st->rel_res   = 0.0;
         x_out();
         MI_HIP(hipStreamSynchronize(s));
-        return MI_OK;
+        return true;
     }
 
     const LocalPreconditioner* fused = nullptr;
@@ -1617,8 +1620,10 @@ extern "C" int mi_pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pc
 
     // a small system's iterations run in one launch (pcg_small.hip) when its
     // preconditioner is one that it knows
-    bool     one_launch = o.use_graph && !ordered && pcg_small_enabled();
+    bool     one_launch = o.use_graph && !ordered && !sys->one_launch_off && pcg_small_enabled();
     SmallPcg sm;
+    if(sys->one_launch_wait >= 0)
+        sm.wait_ticks = sys->one_launch_wait;
     if(one_launch)
     {
         const BsrMatrix& A = sys->A;
@@ -1648,11 +1653,12 @@ extern "C" int mi_pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pc
     }
     while(one_launch && done < total && (sys->one_launch_max < 0 || sys->one_launch_done < sys->one_launch_max))
     {
-        if(!pcg_small_launch(sm, sys->small, total - done, s))
+        if(!pcg_small_launch(sm, sys->small, total - done, o.x_init && sys->one_launch_done == 0, s))
             break;
         ++sys->one_launch_done;
         read_scalars(sys, s);
-        MI_REQUIRE(!h.stalled, MI_ERR_HIP, "mi_pcg_solve: a wait between workgroups ran out");
+        if(h.stalled)
+            return false;
         MI_REQUIRE(std::isfinite(h.rz_new), MI_ERR_NONFINITE,
                    "mi_pcg_solve: non-finite r^T z at iteration " + std::to_string(h.iter));
         done = h.iter;
@@ -1730,6 +1736,33 @@ extern "C" int mi_pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pc
         double rn = norm_f64_host(sys->tmp.data(), n, s);
         double bn = std::sqrt(bb);
         st->rel_res_true = bn > 0 ? rn / bn : 0.0;
+    }
+    return true;
+}
+}  // namespace
+
+extern "C" int mi_pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pcg_opts* opts, mi_pcg_stats* st, void* stream)
+{
+    MI_API_BEGIN
+    MI_REQUIRE(sys && b && x && st, MI_ERR_ARG, "mi_pcg_solve: null argument");
+    MI_REQUIRE(sys->assembled, MI_ERR_STATE, "mi_pcg_solve: system not assembled");
+    MI_REQUIRE(sys->pcs.empty() || sys->pcs_assembled, MI_ERR_STATE, "mi_pcg_solve: preconditioners not assembled");
+    mi_pcg_opts o;
+    mi_pcg_default_opts(&o);
+    if(opts)
+        o = *opts;
+    MI_REQUIRE(o.tol > 0.0 && o.max_iter_ratio > 0.0, MI_ERR_ARG, "mi_pcg_solve: tol and max_iter_ratio must be > 0");
+    MI_REQUIRE(o.criterion == MI_CRIT_RZ_RATIO || o.criterion == MI_CRIT_REL_RESIDUAL, MI_ERR_ARG,
+               "mi_pcg_solve: unknown criterion");
+    hipStream_t s = pick(sys->ctx, stream);
+    if(!pcg_solve(sys, b, x, o, st, s))
+    {
+        // the workgroups did not run at the same time (another process's cooperative
+        // launch holds a part of the CUs): by launches, now and later
+        sys->one_launch_off = true;
+        if(o.x_init)
+            copy_f64(x, sys->small.x0.data(), sys->n(), s);
+        MI_REQUIRE(pcg_solve(sys, b, x, o, st, s), MI_ERR_HIP, "mi_pcg_solve: a wait between workgroups ran out");
     }
     MI_API_END
 }

@@ -682,15 +682,20 @@ struct SmallPcg
     uint64_t* words = nullptr;
     double *  z = nullptr, *pb = nullptr, *R = nullptr, *RA = nullptr, *Z = nullptr;
     int32_t   max_it = 0;
+    // how long a workgroup waits for the others, in ticks of the 100 MHz clock
+    int64_t wait_ticks = 400000000;
 };
 struct SmallPcgScratch
 {
     DBuf<uint64_t> words;
     DBuf<double>   z, pb, R, Z;
+    DBuf<double>   x0;  // the given x of a solve from x0
 };
-// up to max_it iterations from the state in `a`; false when this system, or
-// this device, cannot run them so (nothing is launched then)
-bool pcg_small_launch(SmallPcg& a, SmallPcgScratch& scr, int64_t max_it, hipStream_t s);
+// up to max_it iterations from the state in `a` (keep_x: x is copied to scr.x0
+// first); false when this system, or this device, cannot run them so (nothing
+// is written then).  PcgScalars::stalled is set when a wait ran out: x, r and p may
+// then be those of different iterations.
+bool pcg_small_launch(SmallPcg& a, SmallPcgScratch& scr, int64_t max_it, bool keep_x, hipStream_t s);
 
 // allocates the PCG reductions' partials (must run before any pointer into them is taken)
 void pcg_prepare(SpmvScratch& scr);

@@ -32,8 +32,9 @@
 // seen all of epoch e + 1, which every workgroup stores after it has read all
 // of epoch e.
 //
-// The cooperative launch guarantees that all workgroups are resident; a wait
-// ends after kWaitTicks all the same, and the solve reports it.
+// The cooperative launch guarantees that all workgroups are resident, within one
+// process; a wait ends after a time (4 s) all the same, and the caller then solves
+// again from its start by launches.
 #include <algorithm>
 
 #include "linsys.hpp"
@@ -53,7 +54,6 @@ constexpr int      kBitWords  = kSmallRows / 32;
 constexpr int      kLvl       = 5;              // coarse levels
 constexpr int      kBank      = 16;
 constexpr int      kSym       = 136;
-constexpr uint64_t kWaitTicks = 400000000ull;   // 4 s of the 100 MHz clock
 static_assert(kMaxWg <= 256, "one polled workgroup per thread of four waves");
 
 __device__ __forceinline__ void put(double* p, double v)
@@ -94,7 +94,8 @@ struct Exchange
     uint64_t* words;  // 2 buffers of kMaxWg x 4
     uint32_t  epoch = 0;
     int       wgs, me;
-    double (*red)[4][2];  // LDS, by epoch parity
+    int64_t   wait_ticks;  // of the 100 MHz clock; 0: a wait ends at its first look
+    double (*red)[4][2];   // LDS, by epoch parity
     int* failed;          // LDS
 
     // NV values summed over the workgroups in their order; false when a wait
@@ -143,7 +144,7 @@ struct Exchange
                     }
                 if(__all(ok))
                     break;
-                if((spin & 255u) == 255u && wall_clock64() - start > kWaitTicks)
+                if(wait_ticks == 0 || ((spin & 255u) == 255u && wall_clock64() - start > (uint64_t)wait_ticks))
                 {
                     *failed = 1;
                     break;
@@ -175,14 +176,19 @@ struct Exchange
     }
 };
 
-// clears the exchange words and the restricted r and Ap (nodes no vertex feeds stay 0)
-__global__ void pcg_small_clear_kernel(uint64_t* words, int64_t nwords, double* R, int64_t nr)
+// clears the exchange words and the restricted r and Ap (nodes no vertex feeds
+// stay 0); copies x to x0 where a solve that starts from it may have to start again
+__global__ void pcg_small_clear_kernel(uint64_t* words, int64_t nwords, double* R, int64_t nr, const double* x,
+                                       double* x0, int64_t n)
 {
     const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, st = (int64_t)gridDim.x * blockDim.x;
     for(int64_t i = i0; i < nwords; i += st)
         words[i] = 0ull;
     for(int64_t i = i0; i < nr; i += st)
         R[i] = 0.0;
+    if(x0)
+        for(int64_t i = i0; i < n; i += st)
+            x0[i] = x[i];
 }
 
 // VT: the matrix values; IT: the MAS inverses; MAS: else 3x3 block Jacobi on
@@ -367,7 +373,7 @@ __global__ __launch_bounds__(kNT) void pcg_small_kernel(SmallPcg a)
     bool         conv = false;
     int          it   = 0;
     __syncthreads();
-    Exchange ex{a.words, 0u, (int)gridDim.x, wg, xred, &failed};
+    Exchange ex{a.words, 0u, (int)gridDim.x, wg, a.wait_ticks, xred, &failed};
     // waves that share a node of this workgroup's coarse cluster, above level 1: 2^wsh
     // (one wave per node summed the top cluster's single node in 14 serial rounds,
     // 21.4 us per iteration on 24^3 + 60k against 15.9)
@@ -708,7 +714,7 @@ const void* small_kernel(const SmallPcg& a)
 }
 }  // namespace
 
-bool pcg_small_launch(SmallPcg& a, SmallPcgScratch& scr, int64_t max_it, hipStream_t s)
+bool pcg_small_launch(SmallPcg& a, SmallPcgScratch& scr, int64_t max_it, bool keep_x, hipStream_t s)
 {
     const int     wgs = (a.slots + kRows - 1) / kRows;
     const int64_t n   = 3 * (int64_t)a.B;
@@ -726,7 +732,10 @@ bool pcg_small_launch(SmallPcg& a, SmallPcgScratch& scr, int64_t max_it, hipStre
     a.RA     = a.R + 3 * a.nodes;
     a.Z      = scr.Z.data();
     a.max_it = (int32_t)std::min<int64_t>(max_it, 512);
-    pcg_small_clear_kernel<<<32, 256, 0, s>>>(a.words, 2 * kMaxWg * 4, a.R, a.slot_vec ? 6 * a.nodes : 0);
+    if(keep_x)
+        scr.x0.resize((size_t)n);
+    pcg_small_clear_kernel<<<32, 256, 0, s>>>(a.words, 2 * kMaxWg * 4, a.R, a.slot_vec ? 6 * a.nodes : 0, a.x,
+                                              keep_x ? scr.x0.data() : nullptr, n);
     void*            args[] = {&a};
     const hipError_t e      = hipLaunchCooperativeKernel(small_kernel(a), dim3(wgs), dim3(kNT), args, 0, s);
     if(e != hipSuccess)

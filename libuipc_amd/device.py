@@ -251,6 +251,10 @@ class LinearSystem:
         """the most cooperative launches a solve uses (-1: no limit, 0: the graph)"""
         check(self.lib.mi_sys_set_one_launch(self.h, int(max_launches)))
 
+    def set_one_launch_wait(self, microseconds: int) -> None:
+        """how long a cooperative launch's workgroups wait for each other (-1: 4 s)"""
+        check(self.lib.mi_sys_set_one_launch_wait(self.h, int(microseconds)))
+
     def one_launch(self) -> int:
         """the cooperative launches of the last solve"""
         n = C.c_int32()

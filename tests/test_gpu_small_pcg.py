@@ -148,3 +148,41 @@ def test_small_pcg_goes_on_with_the_graph(ctx, precision, pre):
         # which the launches have too; CG's rounding spreads it by a small factor
         assert st["rel_res_true"] < max(1e-5 * 1.01, 3.0 * graph["rel_res_true"])
     ls.close()
+
+
+@pytest.mark.parametrize("pre", ["diag3", "mas"])
+@pytest.mark.parametrize("x_init", [0, 1])
+def test_small_pcg_wait_runs_out(ctx, pre, x_init):
+    """waits that end at their first look, so that the launch gives up: the solve
+    starts again on the graph, from b and the given x0, and the system stays
+    there until a setter is called"""
+    s = synth.fem_system(9, 0, seed=2)
+    ls = LinearSystem(ctx, s.block_rows)
+    ls.assemble(ctx.to_device(s.rows), ctx.to_device(s.cols), ctx.to_device(s.vals))
+    if pre == "mas":
+        ls.add_preconditioner(abi.MI_PRECOND_MAS, 0, s.n, part_ids=s.part_ids, tets=s.tets)
+    else:
+        ls.add_preconditioner(abi.MI_PRECOND_DIAG3, 0, s.n)
+    ls.assemble_preconditioners()
+    b = ctx.to_device(s.rhs)
+    x0 = np.random.default_rng(5).standard_normal(s.n)
+
+    def solve():
+        x = ctx.to_device(x0)
+        st = ls.solve(b, x, criterion=abi.MI_CRIT_REL_RESIDUAL, tol=1e-8, x_init=x_init, true_residual=1)
+        assert st["converged"] == 1 and st["rel_res_true"] < 1.01e-8
+        return st, x.numpy()
+
+    ls.set_one_launch(0)
+    want, xw = solve()
+    ls.set_one_launch(-1)
+    ls.set_one_launch_wait(0)
+    for _ in range(2):  # the one that gives up, and the next one
+        st, x = solve()
+        assert ls.one_launch() == 0
+        # the same kernels on the same inputs; the MAS sums have no fixed order
+        assert st["iters_exact"] == want["iters_exact"] and rel_err(x, xw) < 1e-9
+    ls.set_one_launch_wait(-1)
+    st, x = solve()
+    assert ls.one_launch() == 1 and rel_err(x, xw) < 1e-6
+    ls.close()
