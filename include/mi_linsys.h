@@ -476,8 +476,7 @@ typedef struct mi_pcg_opts
     int32_t use_graph;      /* 1: replay a captured hipGraph of graph_checks check intervals, or, up to
                              * 16,384 block rows on the full BSR in the caller's vector order with
                              * one DIAG3 or whole-vector MAS or no preconditioner, run the iterations
-                             * in one cooperative launch (mi_sys_set_one_launch; env MI_PCG_SMALL=0:
-                             * always the graph) */
+                             * in one cooperative launch (mi_sys_set_one_launch) */
     int32_t psd_fallback;   /* 1: rz0 < 0 or non-finite -> plain CG (linear_fused_pcg.cu:1843-1875) */
     int32_t force_bypass;   /* 1: always bypass the preconditioner (UIPC_PCG_PSD_FALLBACK_TEST) */
     int32_t true_residual;  /* 1: compute ||b - A x|| / ||b|| after the solve (one SpMV)    */

@@ -1415,16 +1415,6 @@ void run_iteration(mi_sys* sys, double* x, bool bypass, const LocalPreconditione
     pcg_update_p(sc, partB, gB, sys->p.data(), sys->z.data(), n, p32, s);
 }
 
-// MI_PCG_SMALL=0 keeps small systems on the launches of run_iteration
-bool pcg_small_enabled()
-{
-    static const bool on = [] {
-        const char* e = std::getenv("MI_PCG_SMALL");
-        return !(e && std::string(e) == "0");
-    }();
-    return on;
-}
-
 void read_scalars(mi_sys* sys, hipStream_t s)
 {
     MI_HIP(hipMemcpyAsync(sys->h_sc, sys->d_sc, sizeof(PcgScalars), hipMemcpyDeviceToHost, s));
@@ -1620,7 +1610,7 @@ bool pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pcg_opts& o, mi
 
     // a small system's iterations run in one launch (pcg_small.hip) when its
     // preconditioner is one that it knows
-    bool     one_launch = o.use_graph && !ordered && !sys->one_launch_off && pcg_small_enabled();
+    bool     one_launch = o.use_graph && !ordered && !sys->one_launch_off;
     SmallPcg sm;
     if(sys->one_launch_wait >= 0)
         sm.wait_ticks = sys->one_launch_wait;
