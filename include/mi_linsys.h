@@ -527,6 +527,9 @@ int mi_pcg_solve(mi_sys*            sys,
  * uses before it goes on with the captured graph; -1 (the default): no limit,
  * 0: the graph from the start.  mi_sys_one_launch: how many the last solve used
  * (0: it ran on the graph or on plain launches).
+ * A workgroup takes 64 rows (with a MAS 64 partition slots, of which there may be
+ * 16,384 too).  Systems where one would hold far more blocks than the others, a
+ * few dense rows next to each other, go to the graph.
  * The launch's workgroups wait for each other.  Where a wait runs out (they do not
  * all run, as when another process holds a part of the GPU in the same way), the
  * solve starts again on the graph, and the system stays on it until one of the

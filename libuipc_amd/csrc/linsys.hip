@@ -110,6 +110,7 @@ struct mi_sys
     int64_t         one_launch_wait = -1;  // ticks that a workgroup waits (-1: the default)
     int32_t         one_launch_done = 0;   // launches of the last solve
     bool            one_launch_off  = false;  // a wait ran out: the graph from then on
+    bool            one_launch_unfit[2] = {};  // the assembled rows do not suit it, split in the caller's order, by the MAS
 
     // batched solves (mi_pcg_solve_batched): the tile table of the last
     // segmentation, per-system scalars, tile partials and their own graph
@@ -470,6 +471,7 @@ void assemble_t(mi_sys* sys, int64_t T, const int32_t* rows, const int32_t* cols
     build_spmv_layout(sys, s);
     sys->assembled     = true;
     sys->pcs_assembled = false;
+    sys->one_launch_unfit[0] = sys->one_launch_unfit[1] = false;
 }
 }  // namespace
 
@@ -874,6 +876,7 @@ int mi_precond_add(mi_sys* sys, const mi_precond_desc* d, int* handle)
     auto pc = build_precond(sys, d, -1, "mi_precond_add");
     sys->pcs.push_back(std::move(pc));
     sys->pcs_assembled = false;
+    sys->one_launch_unfit[0] = sys->one_launch_unfit[1] = false;
     ++sys->pcs_gen;
     ++sys->order_gen;
     if(handle)
@@ -889,6 +892,7 @@ int mi_precond_reinit(mi_sys* sys, int handle, const mi_precond_desc* d)
     MI_HIP(hipDeviceSynchronize());  // no launch may still read the preconditioner being replaced
     sys->pcs[handle]   = std::move(pc);
     sys->pcs_assembled = false;
+    sys->one_launch_unfit[0] = sys->one_launch_unfit[1] = false;
     ++sys->pcs_gen;
     ++sys->order_gen;
     MI_API_END
@@ -1641,12 +1645,17 @@ bool pcg_solve(mi_sys* sys, const double* b, double* x, const mi_pcg_opts& o, mi
                 one_launch = sys->pcs.size() == 1 && sys->pcs[0]->small_pcg(sm);
         }
     }
+    bool& unfit = sys->one_launch_unfit[sm.slot_vec ? 1 : 0];
+    one_launch  = one_launch && !unfit;
     while(one_launch && done < total && (sys->one_launch_max < 0 || sys->one_launch_done < sys->one_launch_max))
     {
         if(!pcg_small_launch(sm, sys->small, total - done, o.x_init && sys->one_launch_done == 0, s))
             break;
-        ++sys->one_launch_done;
         read_scalars(sys, s);
+        unfit = h.stalled == kPcgUnfit;
+        if(unfit)
+            break;
+        ++sys->one_launch_done;
         if(h.stalled)
             return false;
         MI_REQUIRE(std::isfinite(h.rz_new), MI_ERR_NONFINITE,

@@ -478,8 +478,10 @@ struct PcgScalars
     int32_t criterion;
     int32_t iter;
     int32_t conv_iter;
-    int32_t stalled;  // a wait between workgroups ran out (pcg_small_launch)
+    int32_t stalled;  // pcg_small_launch: kPcgStalled, kPcgUnfit
 };
+constexpr int32_t kPcgStalled = 1;  // a wait between workgroups ran out
+constexpr int32_t kPcgUnfit   = 2;  // a workgroup's rows hold too many blocks: nothing was done
 
 // the fixed-order sum of a reduction's partials (stride apart), redone by every
 // workgroup of NT threads of the consuming kernel (no fence, no atomics,
@@ -693,8 +695,8 @@ struct SmallPcgScratch
 };
 // up to max_it iterations from the state in `a` (keep_x: x is copied to scr.x0
 // first); false when this system, or this device, cannot run them so (nothing
-// is written then).  PcgScalars::stalled is set when a wait ran out: x, r and p may
-// then be those of different iterations.
+// is written then).  PcgScalars::stalled: kPcgUnfit, the state is as it was, or
+// kPcgStalled, x, r and p may be those of different iterations.
 bool pcg_small_launch(SmallPcg& a, SmallPcgScratch& scr, int64_t max_it, bool keep_x, hipStream_t s);
 
 // allocates the PCG reductions' partials (must run before any pointer into them is taken)

@@ -35,6 +35,19 @@
 // The cooperative launch guarantees that all workgroups are resident, within one
 // process; a wait ends after a time (4 s) all the same, and the caller then solves
 // again from its start by launches.
+//
+// Rows are split by their count, not by their blocks, so one workgroup may hold
+// what all others wait for.  A launch whose heaviest workgroup is past the limits
+// below gives up before its first iteration (unfit), and the caller takes the
+// launches, whose SpMV is split by blocks.  us per iteration against theirs, by a
+// workgroup's blocks:
+//   2,048 columns or fewer: 7,455 blocks (12^3 + 200k contacts) 30 against 33, 5,726
+//     (8^3 + 100k) 24 (33); 7,649 random ones of 2,048 rows 6.9 (5.5);
+//   more columns: 2,741 blocks (random rows) 7.4 (9.2); 3,223, eight rows of 319
+//     among them, 21.0 (16.5); 16 rows of 2,000 and more together 110 to 1,230
+//     (33 to 117), 64 of 13,000 4,887 (136);
+//   one long row, which is as serial in the launches: of 4,000 blocks 43 to 49
+//     (42 to 57), of 13,000 86 to 102 (108 to 125), two of 1,500 31 (25).
 #include <algorithm>
 
 #include "linsys.hpp"
@@ -50,6 +63,8 @@ constexpr int      kPer       = 3;              // blocks per thread in register
 constexpr int      kStage     = kPer * kNT;     // blocks per stage
 constexpr int      kCols      = 2048;           // columns whose p is kept in LDS
 constexpr int      kMaxWg     = kSmallRows / kRows;
+constexpr int      kFitNear   = 7500;           // blocks of a workgroup whose columns are all in LDS
+constexpr int      kFitLong   = 2048;           // ... beside its longest row, where they are not
 constexpr int      kBitWords  = kSmallRows / 32;
 constexpr int      kLvl       = 5;              // coarse levels
 constexpr int      kBank      = 16;
@@ -247,6 +262,23 @@ __global__ __launch_bounds__(kNT) void pcg_small_kernel(SmallPcg a)
         bits[t] = 0u;
     __syncthreads();
     const int nb      = rs[kRows];
+    int       longest = 0;  // row
+    {
+        int l = t < kRows ? rs[t + 1] - rs[t] : 0;
+        if(t < kRows)
+        {
+#pragma unroll
+            for(int o = kRows / 2; o > 0; o >>= 1)
+                l = max(l, __shfl_xor(l, o, kWave));
+            if(t == 0)
+                lds[0] = (uint32_t)l;
+        }
+        __syncthreads();
+        longest = (int)lds[0];
+        __syncthreads();
+    }
+    // unfit whatever its columns (they need not be looked at then)
+    bool unfit = nb > kFitNear && nb - longest > kFitLong;
     auto      row_of  = [&](int i) {
         int lo = 0;
 #pragma unroll
@@ -255,7 +287,7 @@ __global__ __launch_bounds__(kNT) void pcg_small_kernel(SmallPcg a)
         return lo;
     };
     // ---- the columns it meets: a bit each, numbered in ascending order
-    for(int i = t; i < nb; i += kNT)
+    for(int i = t; i < nb && !unfit; i += kNT)
     {
         const int     row = row_of(i);
         const int32_t j   = a.fcols[rb[row] + (i - rs[row])];
@@ -275,6 +307,7 @@ __global__ __launch_bounds__(kNT) void pcg_small_kernel(SmallPcg a)
         }
     }
     __syncthreads();
+    unfit = unfit || (ncols > (uint32_t)kCols && nb > kStage && nb - longest > kFitLong);
     const int nl = 3 * (int)(ncols < (uint32_t)kCols ? ncols : (uint32_t)kCols);
     // a column's place in pj, or ~column past the ones kept there
     auto local_of = [&](int32_t j) -> int32_t {
@@ -444,20 +477,25 @@ __global__ __launch_bounds__(kNT) void pcg_small_kernel(SmallPcg a)
         }
     };
     double d0 = 0.0, d1 = 0.0;
-    bool   go = true;
+    if(t == 0)
+        wred[0][0][0] = unfit ? 1.0 : 0.0;
     if constexpr(MAS)
     {
         if(t < 3 * kBank)
             sC[t] = 0.0;
-        if(a.levels > 1)
-        {
-            if(t / kOwn == kRows / kBank)
-                restrict1(t, sr, a.R);
-            go = ex.run<0>(wred[0], d0, d1);
-            if(go && coarse_wg)
-                coarse_r(t, a.R, 1.0);
-        }
+        if(a.levels > 1 && t / kOwn == kRows / kBank)
+            restrict1(t, sr, a.R);
     }
+    bool go = ex.run<1, 1>(wred[0], d0, d1);
+    if(go && d0 != 0.0)
+    {
+        if(wg == 0 && t == 0)
+            a.sc->stalled = kPcgUnfit;
+        return;
+    }
+    if constexpr(MAS)
+        if(go && coarse_wg)
+            coarse_r(t, a.R, 1.0);
     while(go && it < a.max_it)
     {
         int t = threadIdx.x;
@@ -671,7 +709,7 @@ __global__ __launch_bounds__(kNT) void pcg_small_kernel(SmallPcg a)
     if(failed)
     {
         if(t == 0)
-            a.sc->stalled = 1;
+            a.sc->stalled = kPcgStalled;
         return;
     }
     int32_t v;

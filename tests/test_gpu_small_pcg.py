@@ -186,3 +186,47 @@ def test_small_pcg_wait_runs_out(ctx, pre, x_init):
     st, x = solve()
     assert ls.one_launch() == 1 and rel_err(x, xw) < 1e-6
     ls.close()
+
+
+@pytest.mark.parametrize("pre", ["diag3", "mas"])
+@pytest.mark.parametrize("hubs,reach,fits", [(1, 0, True), (1, 3900, True), (2, 1500, False), (8, 450, False),
+                                             (60, 900, False)])
+def test_small_pcg_dense_rows(ctx, pre, hubs, reach, fits):
+    """`hubs` rows of one workgroup, each coupled to `reach` others: one long row
+    stays on the one launch, several go to the launches (whose SpMV is split by
+    blocks, not by rows), and so does the system's next solve; after an assembly
+    without them it is on the one launch again"""
+    s = synth.fem_system(16, 0, seed=2)
+    rng = np.random.default_rng(hubs)
+    rows, cols, vals = [s.rows], [s.cols], [s.vals]
+    # rows that share a workgroup in the caller's order and in the partition's
+    hub = np.arange(640, 704)[:hubs] if pre == "diag3" else np.argsort(s.part_ids, kind="stable")[640:640 + hubs]
+    for h in hub.astype(np.int32):
+        j = np.setdiff1d(rng.choice(s.block_rows, reach, replace=False), [h]).astype(np.int32)
+        g = rng.standard_normal((j.size, 3))
+        g /= np.linalg.norm(g, axis=1)[:, None]
+        k = (g[:, :, None] * g[:, None, :]).reshape(-1, 9)
+        at = np.full(j.size, h, np.int32)
+        rows += [at, j, np.minimum(at, j)]
+        cols += [at, j, np.maximum(at, j)]
+        vals += [k, k, -k]
+    ls = LinearSystem(ctx, s.block_rows)
+    keep = [ctx.to_device(np.concatenate(v)) for v in (rows, cols, vals)]
+    ls.assemble(*keep)
+    if pre == "mas":
+        ls.add_preconditioner(abi.MI_PRECOND_MAS, 0, s.n, part_ids=s.part_ids, tets=s.tets)
+    else:
+        ls.add_preconditioner(abi.MI_PRECOND_DIAG3, 0, s.n)
+    ls.assemble_preconditioners()
+    b = ctx.to_device(s.rhs)
+    for _ in range(2):
+        check(ctx, ls, b)
+        x = ctx.alloc(s.n, np.float64)
+        ls.solve(b, x, criterion=abi.MI_CRIT_REL_RESIDUAL, tol=1e-8)
+        assert ls.one_launch() == (1 if fits else 0)
+    free = [ctx.to_device(v) for v in (s.rows, s.cols, s.vals)]
+    ls.assemble(*free)
+    ls.assemble_preconditioners()
+    ls.solve(b, ctx.alloc(s.n, np.float64), criterion=abi.MI_CRIT_REL_RESIDUAL, tol=1e-8)
+    assert ls.one_launch() == 1
+    ls.close()
