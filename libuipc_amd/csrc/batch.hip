@@ -4,10 +4,10 @@
 // FusedPCG (linear_system/linear_fused_pcg.cu:1374-2004) runs once per system
 // in the reference; here one captured iteration serves every system:
 //   the SpMV runs over the union (no block couples two systems);
-//   every dot is a per-system sum: the DoFs are cut into tiles of at most
-//     kTile DoFs that never cross a system boundary (a host-built table), one
-//     workgroup writes each tile's partial, and every wave that needs a
-//     system's sum adds its tiles in order (deterministic, no atomics);
+//   every dot is a per-system sum: the DoFs are cut into tiles that never cross
+//     a system boundary (batch_tile; a host-built table), one workgroup writes
+//     each tile's partial, and every wave or workgroup that needs a system's sum
+//     adds its tiles in a fixed order (deterministic, no atomics);
 //   alpha, beta, the convergence test and the iteration cap are per system;
 //     a system that has converged or reached its cap stops changing;
 //   the x / r and p updates run tile by tile, each tile reading its system's
@@ -27,6 +27,24 @@ __device__ __forceinline__ double wave_tiles(const double* part, int stride, int
     for(int32_t t = t0 + (int32_t)__lane_id(); t < t1; t += kWave)
         acc += part[stride * (int64_t)t];
     return wave_sum(acc);
+}
+
+// the same by every workgroup that calls it: each wave by itself up to 64 tiles
+// (no barrier), else all waves together (lds: 4 values of this sum alone; a wave's own
+// sum took 60.9 us per iteration on a system of 5.9e5 DoFs, 573 tiles, against 56.6)
+__device__ __forceinline__ double group_tiles(const double* part, int32_t t0, int32_t t1, double* lds)
+{
+    if(t1 - t0 <= kWave)
+        return wave_tiles(part, 1, t0, t1);
+    double acc = 0.0;
+    for(int32_t t = t0 + (int32_t)threadIdx.x; t < t1; t += kThreads)
+        acc += part[t];
+    acc = wave_sum(acc);
+    __syncthreads();  // the last tile's sum is read
+    if(threadIdx.x % kWave == 0)
+        lds[threadIdx.x / kWave] = acc;
+    __syncthreads();
+    return (lds[0] + lds[1]) + (lds[2] + lds[3]);
 }
 
 // tile partials of a . b (and of a . a when aa != nullptr)
@@ -112,7 +130,7 @@ __global__ __launch_bounds__(kThreads) void batch_bypass_z_kernel(const BatchTil
 }
 
 // alpha = rz / pAp per system (fused_update_xr's scalar), then x and r.  Every
-// wave sums its system's partials by itself, in the same order; the
+// workgroup sums its system's partials by itself, in the same order; the
 // system's first tile records the scalars (no tile reads those it writes).  A
 // kernel of its own for them was 4.7 us of an iteration's 139 (12 systems of 3e3 to
 // 1e5 DoFs), and so was beta's.
@@ -124,6 +142,7 @@ __global__ __launch_bounds__(kThreads) void batch_update_xr_kernel(const BatchTi
                                                                   double*       r,
                                                                   const double* __restrict__ Ap)
 {
+    __shared__ double lds[kThreads / kWave];
     for(int32_t t = blockIdx.x; t < tiles.n; t += gridDim.x)
     {
         const int32_t g = tiles.sys[t];
@@ -131,7 +150,7 @@ __global__ __launch_bounds__(kThreads) void batch_update_xr_kernel(const BatchTi
         if(q.stopped)
             continue;
         const int32_t t0 = tiles.sys_tile[g];
-        const double  rz = q.rz_pending, v = wave_tiles(pap, 1, t0, tiles.sys_tile[g + 1]);
+        const double  rz = q.rz_pending, v = group_tiles(pap, t0, tiles.sys_tile[g + 1], lds);
         const double  alpha = rz / v;
         if(t == t0 && threadIdx.x == 0)
         {
@@ -161,14 +180,28 @@ __global__ __launch_bounds__(kThreads) void batch_update_p_kernel(const BatchTil
                                                                  const double* __restrict__ z,
                                                                  float4*       p32)
 {
+    __shared__ double  lds[2][kThreads / kWave];
+    __shared__ int32_t stop;
     for(int32_t t = blockIdx.x; t < tiles.n; t += gridDim.x)
     {
         const int32_t g = tiles.sys[t];
         BatchScalars& q = sc[g];
-        if(__hip_atomic_load(&q.stopped, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            continue;
         const int32_t t0 = tiles.sys_tile[g], t1 = tiles.sys_tile[g + 1];
-        const double  rz_new = wave_tiles(rz, 1, t0, t1), rr_new = wave_tiles(rr, 1, t0, t1);
+        int32_t       off = 0;
+        if(t1 - t0 <= kWave)
+            off = __hip_atomic_load(&q.stopped, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else
+        {
+            // once for the workgroup, whose waves meet below: the mark may be set meanwhile
+            __syncthreads();
+            if(threadIdx.x == 0)
+                stop = __hip_atomic_load(&q.stopped, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            off = stop;
+        }
+        if(off)
+            continue;
+        const double  rz_new = group_tiles(rz, t0, t1, lds[0]), rr_new = group_tiles(rr, t0, t1, lds[1]);
         const double  beta = rz_new / q.rz;
         bool          conv = q.criterion == 0 ? (fabs(rz_new) <= q.rz_tol) : (rr_new <= q.rr_tol);
         if(!isfinite(rz_new) || !isfinite(rr_new))

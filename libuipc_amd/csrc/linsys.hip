@@ -1807,9 +1807,9 @@ std::vector<double> host_seg_sums(mi_sys* sys, const double* part, int32_t nseg,
     int32_t             t = 0;
     for(int32_t g = 0; g < nseg; ++g)
     {
-        const int64_t hi = 3 * (int64_t)bt.seg_rows[g + 1];
+        const int64_t hi = 3 * (int64_t)bt.seg_rows[g + 1], step = batch_tile(bt.seg_rows[g + 1] - bt.seg_rows[g]);
         double        acc = 0.0;
-        for(int64_t lo = 3 * (int64_t)bt.seg_rows[g]; lo < hi; lo += kBatchTile)
+        for(int64_t lo = 3 * (int64_t)bt.seg_rows[g]; lo < hi; lo += step)
             acc += bt.h_part[t++];
         out[g] = acc;
     }
@@ -1858,8 +1858,8 @@ extern "C" int mi_pcg_solve_batched(mi_sys*            sys,
         {
             stile[g]        = (int32_t)lo.size();
             slo[g]          = 3 * (int64_t)seg_rows[g];
-            const int64_t e = 3 * (int64_t)seg_rows[g + 1];
-            for(int64_t t = slo[g]; t < e; t += kBatchTile)
+            const int64_t e = 3 * (int64_t)seg_rows[g + 1], step = batch_tile(seg_rows[g + 1] - seg_rows[g]);
+            for(int64_t t = slo[g]; t < e; t += step)
             {
                 lo.push_back(t);
                 tsys.push_back(g);

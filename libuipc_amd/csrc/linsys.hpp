@@ -596,12 +596,23 @@ __device__ __forceinline__ double pcg_alpha_of(PcgScalars* sc, const double* pap
 }
 
 // ---- batched PCG: independent systems on consecutive block-row ranges
-// Tiles of at most kBatchTile DoFs (whole block rows) that never cross a
-// system boundary; every per-system sum runs over its tiles in order.
+// Tiles of kBatchTile DoFs (whole block rows) that never cross a system
+// boundary; every per-system sum runs over its tiles in order.
 // 1,023 DoFs give each of a workgroup's lanes four: 12 systems of 3e3 to 1e5 DoFs are
 // 420 tiles (with 4,095, 105: fewer workgroups than CUs; the dots 6.3 -> 4.7 us, x and r
 // 8.7 -> 5.3 with alpha's sum in it)
 constexpr int64_t kBatchTile = 3 * 341;
+// A system has at most kBatchTiles tiles, larger ones past 1e6 DoFs: every tile of
+// the x, r and p updates adds up all of its system's partials, so their reads grow
+// with the square of the tiles.  us per iteration of one system of 6e6 / 1.2e7 DoFs:
+// any number of tiles 583 / 1,573 (tiles of 4,095 and a kernel for the sums 404 /
+// 804), at most 2,048 392 / 773, 1,024 386 / 764, 512 409 / 845, 256 467 / 1,015
+constexpr int64_t kBatchTiles = 1024;
+// the DoFs per tile of a system of this many block rows
+inline int64_t batch_tile(int64_t rows)
+{
+    return std::max<int64_t>(kBatchTile, 3 * ((rows + kBatchTiles - 1) / kBatchTiles));
+}
 // ----------------------------------------------------------------- learned initial guess
 void ws_gemm(int32_t M, int32_t N, int32_t K, const float* A, int64_t sa_m, int64_t sa_k, const float* B,
              int64_t sb_k, int64_t sb_n, float* C, int64_t ldc, bool accumulate, const float* bias, bool relu,

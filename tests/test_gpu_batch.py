@@ -275,3 +275,66 @@ def test_batch_tile_edges(ctx, sizes, kind):
         want = np.linalg.solve(A, rhs.reshape(B, 3)[seg[k]:seg[k + 1]])
         assert sts[k]["converged"] == 1 and rel_err(xs[seg[k]:seg[k + 1]], want) < 1e-9, (k, n, sts[k])
     ls.close()
+
+
+def chains(ctx, sizes):
+    """systems of `sizes` block rows, each a chain with blocks 3I on the diagonal
+    and -I beside it, with the 3x3 block Jacobi"""
+    seg = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    B = int(seg[-1])
+    diag = np.arange(B, dtype=np.int32)
+    links = np.delete(diag[:-1], seg[1:-1] - 1)
+    rows, cols = np.concatenate([diag, links]), np.concatenate([diag, links + np.int32(1)])
+    vals = np.concatenate([np.tile(3 * np.eye(3).ravel(), (B, 1)), np.tile(-np.eye(3).ravel(), (links.size, 1))])
+    ls = LinearSystem(ctx, B)
+    ls.assemble(ctx.to_device(rows), ctx.to_device(cols), ctx.to_device(vals))
+    ls.add_preconditioner(abi.MI_PRECOND_DIAG3, 0, 3 * B)
+    ls.assemble_preconditioners()
+    return ls, seg
+
+
+@pytest.mark.parametrize("sizes", [[341 * 64, 341 * 64 + 1, 5], [341 * 1024, 341 * 1024 + 1, 2], [1200007, 30]],
+                         ids=lambda s: "-".join(map(str, s)))
+def test_batch_many_tiles(ctx, sizes):
+    """systems of 64 and 65 tiles (a sum by each wave, by the workgroup), of 1,024
+    tiles and past them (longer tiles): test_batch_tile_edges' chains and bounds"""
+    from scipy.linalg import solveh_banded
+
+    ls, seg = chains(ctx, sizes)
+    rhs = np.random.default_rng(7).standard_normal(3 * int(seg[-1]))
+    x = ctx.alloc(rhs.size, np.float64)
+    sts = ls.solve_batched(seg, ctx.to_device(rhs), x, criterion=abi.MI_CRIT_REL_RESIDUAL, tol=1e-10,
+                           max_iter_ratio=100.0)
+    xs = x.numpy().reshape(-1, 3)
+    for k, n in enumerate(sizes):
+        band = np.stack([np.full(n, -1.0), np.full(n, 3.0)])
+        want = solveh_banded(band, rhs.reshape(-1, 3)[seg[k]:seg[k + 1]])
+        assert sts[k]["converged"] == 1 and rel_err(xs[seg[k]:seg[k + 1]], want) < 1e-9, (k, n, sts[k])
+    ls.close()
+
+
+def test_batch_large_system_time(ctx):
+    """the same 2,000,000 rows as one system and as eight: the sums of one large
+    system must not grow with the square of its tiles (20.4 ms against
+    12.4 when they did, now 12.4 against 12.7)"""
+    n = 250_000
+    ls, seg = chains(ctx, [n] * 8)
+    b = ctx.to_device(np.random.default_rng(7).standard_normal(3 * int(seg[-1])))
+    x = ctx.alloc(3 * int(seg[-1]), np.float64)
+
+    def seconds(s):
+        best = 1e9
+        for _ in range(4):
+            ctx.synchronize()
+            t = time.perf_counter()
+            st = ls.solve_batched(s, b, x, criterion=abi.MI_CRIT_REL_RESIDUAL, tol=1e-300,
+                                  max_iter_ratio=41.5 / (3.0 * (s[1] - s[0])))
+            ctx.synchronize()
+            best = min(best, time.perf_counter() - t)
+        assert all(q["iters"] == 41 for q in st)
+        return best
+
+    eight, one = seconds(seg), seconds(seg[[0, -1]])
+    print(f"one system of 6e6 DoFs: {one * 1e3:.2f} ms, eight {eight * 1e3:.2f}", flush=True)
+    assert one < 1.25 * eight
+    ls.close()
