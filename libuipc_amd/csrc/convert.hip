@@ -20,6 +20,7 @@
 //     of the off-diagonal blocks) and merged row by row into a full BSR, so the
 //     SpMV is a pure row gather without atomics.
 #include "linsys.hpp"
+#include "segtile.hpp"
 
 namespace mi
 {
@@ -496,9 +497,6 @@ __global__ __launch_bounds__(kThreads) void rle_count_kernel(const int64_t* d_m,
         tile_cnt[blockIdx.x] = s;
 }
 
-constexpr int kSegTile = 256;  // sorted entries per tile of the segmented reduce
-constexpr int kSegTail = 96;   // entries past the tile staged with it
-
 template <typename KeyT>
 __global__ __launch_bounds__(kThreads) void rle_write_kernel(const int64_t*  d_m,
                                                             const KeyT*     keys,
@@ -590,9 +588,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     __shared__ TV      sv[9 * kCap];
     __shared__ int32_t ss[2][kCap];
     __shared__ int32_t sb[2][kSegTile + 1];
-    const int32_t m   = (int32_t)*d_m;
-    const int32_t nt  = (m + kSegTile - 1) / kSegTile;
-    const int     tid = threadIdx.x;
+    const uint32_t m   = (uint32_t)*d_m;
+    const int32_t  nt  = (int32_t)seg_tiles(m);
+    const int      tid = threadIdx.x;
     auto tile_of = [&](int64_t k) -> int32_t {  // the workgroup's k-th tile (nt: none)
         const int64_t t = k * gridDim.x + blockIdx.x;
         return t < nt ? (int32_t)t : nt;
@@ -605,11 +603,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         hu1 = t < nt ? (t + 1 < nt ? seg_tile[t + 1] : (uint32_t)U) : 0;
     };
     auto index_load = [&](int32_t t) {  // uses hu0, hu1 of t
-        const int32_t e = t * kSegTile + tid;
+        const uint32_t e = seg_entry((uint32_t)t, tid), et = seg_entry((uint32_t)t, kSegTile + tid);
         i_src  = e < m ? srcs[e] : 0;
-        i_tail = tid < kSegTail && e + kSegTile < m ? srcs[e + kSegTile] : 0;
-        i_sb   = hu0 + tid < hu1 ? seg_start[hu0 + tid] : m;
-        i_end  = hu1 < U ? seg_start[hu1] : m;
+        i_tail = tid < kSegTail && et < m ? srcs[et] : 0;
+        i_sb   = hu0 + tid < hu1 ? seg_start[hu0 + tid] : (int32_t)m;
+        i_end  = hu1 < U ? seg_start[hu1] : (int32_t)m;
     };
     auto index_store = [&](int s, int nb) {
         ss[s][tid] = i_src;
