@@ -830,6 +830,12 @@ int spmv_default_shape()
 //   FP32: 33^3 12.4 (15.3), 37^3 + 300k 16.9 (22.7); 41^3 one block per load
 //         21.6 (27.1), 46^3 + 500k 25.4 (27.6); 52^3 four blocks per load 37.6
 //         (46.8); 61^3 512 rows 55.6, 64^3 + 2M 64.1 (256 on 128: 59.5, 69.2)
+// 128-row windows end where five workgroups per CU, all that fit, no longer hold
+// them in one round: whole PCG iterations at 54^3 + 1.2M (1,231 windows) FP64 113.7
+// (256-row windows 120.2), FP32 82.9 (92.3), at 55^3 + 1.3M (1,300) 126.9 (121.7) and 103.3
+// (93.5), 57^3 + 0.4M FP32 85.7 (79.4).  FP64 64-row windows end for the same reason at
+// 81,920 rows: 43^3 + 0.6M 72.4 (128 rows: 75.6), 44^3 + 0.65M 76.3 (75.3), until their
+// second round is well filled too, 48^3 + 0.84M 87.5 (88.7).
 // In the caller's order (no MAS) the same choices measured 19.0 (21.8), 35.9
 // (40.9) and 71.2 (78.5) in FP64.  Up to 16,384 rows the full BSR's row
 // gather is as fast (20^3: 5.8 against 9.1) or near (25^3 + 90k: 12.0
@@ -843,8 +849,9 @@ int spmv_auto_shape(int64_t B, bool use32)
         int64_t rows;  // from this many block rows on
         int     f64, f32;
     };
-    // rows per CU (256 of them): 768, 448, 224 or 160, 64
-    static constexpr Rule rules[] = {{196608, 0, 11}, {114688, 15, 16}, {57344, 13, 14}, {40960, 13, 12}, {16385, 12, 12}};
+    // rows per CU (256 of them): 768, 640, 448, 384, 320, 224, 160, 64
+    static constexpr Rule rules[] = {{196608, 0, 11}, {163841, 3, 3},  {114688, 15, 16}, {98304, 13, 14},
+                                     {81921, 15, 14}, {57344, 13, 14}, {40960, 13, 12},  {16385, 12, 12}};
     const int64_t         rows    = B * 256 / std::max(1, device_cu_count());
     for(const Rule& r : rules)
         if(rows >= r.rows)

@@ -302,6 +302,20 @@ def test_spmv_every_launch_shape(ctx, c1_contact, precision):
     ls.close()
 
 
+@pytest.mark.parametrize("B,rows", [(16384, (0, 0)), (57344, (64, 64)), (81920, (64, 64)), (81921, (128, 64)),
+                                    (98304, (64, 64)), (114687, (64, 64)), (114688, (128, 128)), (163840, (128, 128)),
+                                    (163841, (256, 256)), (196607, (256, 256)), (196608, (512, 512))])
+def test_spmv_windows_by_size(ctx, B, rows):
+    """the window sizes at the lines of the rule (FP64, FP32)"""
+    for precision, want in zip((abi.MI_FP64, abi.MI_FP32), rows):
+        ls = LinearSystem(ctx, B, precision)
+        i = np.arange(B, dtype=np.int32)
+        ls.assemble(ctx.to_device(i), ctx.to_device(i), ctx.to_device(np.tile(np.eye(3).ravel(), (B, 1))))
+        lay = ls.spmv_layout()
+        assert lay["window_rows"] == want and lay["layout"] == ("window" if want else "full")
+        ls.close()
+
+
 @pytest.mark.parametrize("precision", [abi.MI_FP64, abi.MI_FP32])
 @pytest.mark.parametrize("grid,rows", [(25, 0), (26, 64), (39, 64)])
 def test_spmv_layout_by_size(ctx, precision, grid, rows):
