@@ -215,10 +215,14 @@ int mi_spmv_shapes(int32_t* count, int32_t* dflt, int32_t* threads, int32_t* row
 enum
 {
     MI_SPMV_SHAPE_AUTO = -1, /* by the system's size (the default): windows small enough to fill the
-                                GPU with workgroups, from 64 rows above 16,384 block rows to 512
-                                rows; the full BSR up to 16,384 block rows                     */
+                                GPU with workgroups, from 64 rows above 16,384 block rows (without
+                                a MAS, 49,151) to 512 rows; the full BSR up to there           */
     MI_SPMV_SHAPE_FULL = -2  /* the full BSR (both triangles, a row gather)                       */
 };
+/* The full BSR sums every row in a fixed order: a product is the same bits in
+ * every run, and so is a solve without a MAS (which sums by atomics itself).  On a
+ * window layout the products of a window's blocks are added in the order they come,
+ * so results differ between runs by rounding; MI_SPMV_SHAPE_FULL restores the order. */
 /* The layout this system's SpMV uses: a window shape (an index of
  * mi_spmv_shapes), MI_SPMV_SHAPE_AUTO or MI_SPMV_SHAPE_FULL.  An assembled
  * system gets the new layout at once, on `stream`. */

@@ -197,8 +197,22 @@ static int layout_shape(const mi_sys* sys)
     if(!spmv_use_window())
         return spmv_shape_full;
     if(sys->spmv_shape == spmv_shape_auto)
-        return spmv_auto_shape(sys->desc.block_rows, sys->desc.value_precision == MI_FP32);
+    {
+        const bool part_order = std::any_of(sys->pcs.begin(), sys->pcs.end(),
+                                            [](const auto& pc) { return pc->spmv_rank() != nullptr; });
+        return spmv_auto_shape(sys->desc.block_rows, sys->desc.value_precision == MI_FP32, part_order);
+    }
     return sys->spmv_shape;
+}
+
+// does the assembled matrix hold another layout than it should now (another
+// shape was chosen, a preconditioner has come or gone)?
+static bool layout_stale(const mi_sys* sys)
+{
+    const int want = layout_shape(sys);
+    if(want < 0)
+        return sys->A.has_win;
+    return !sys->A.has_win || sys->A.wshape != want || sys->A.win_order != sys->order_gen;
 }
 
 // the SpMV's layout of the assembled matrix: the full BSR (built from the
@@ -726,8 +740,7 @@ int mi_sys_set_spmv_shape(mi_sys* sys, int32_t shape, void* stream)
                MI_ERR_ARG, "mi_sys_set_spmv_shape: unknown shape");
     sys->spmv_shape = shape;
     // an assembled system gets the new layout at once
-    const int want = layout_shape(sys);
-    if(sys->assembled && (want < 0 ? sys->A.has_win : (!sys->A.has_win || sys->A.wshape != want)))
+    if(sys->assembled && layout_stale(sys))
         build_spmv_layout(sys, pick(sys->ctx, stream));
     MI_API_END
 }
@@ -932,8 +945,8 @@ int mi_precond_assemble(mi_sys* sys, void* stream)
     MI_REQUIRE(sys, MI_ERR_ARG, "null sys");
     MI_REQUIRE(sys->assembled, MI_ERR_STATE, "mi_precond_assemble: assemble the system first");
     hipStream_t s = pick(sys->ctx, stream);
-    // a preconditioner added since the assembly may change the SpMV's row order
-    if(sys->A.has_win && sys->A.win_order != sys->order_gen)
+    // a preconditioner added since the assembly may change the SpMV's layout or row order
+    if(layout_stale(sys))
         build_spmv_layout(sys, s);
     for(auto& pc : sys->pcs)
         pc->assemble(sys->A, s);

@@ -836,11 +836,14 @@ int spmv_default_shape()
 // (93.5), 57^3 + 0.4M FP32 85.7 (79.4).  FP64 64-row windows end for the same reason at
 // 81,920 rows: 43^3 + 0.6M 72.4 (128 rows: 75.6), 44^3 + 0.65M 76.3 (75.3), until their
 // second round is well filled too, 48^3 + 0.84M 87.5 (88.7).
-// In the caller's order (no MAS) the same choices measured 19.0 (21.8), 35.9
-// (40.9) and 71.2 (78.5) in FP64.  Up to 16,384 rows the full BSR's row
-// gather is as fast (20^3: 5.8 against 9.1) or near (25^3 + 90k: 12.0
-// against 10.1), and its sums do not depend on scheduling.
-int spmv_auto_shape(int64_t B, bool use32)
+// In the caller's order (no MAS) the same choices measured 35.9 (40.9) and 71.2
+// (78.5) in FP64.  Up to 16,384 rows the full BSR's row gather is as fast (20^3: 5.8
+// against 9.1) or near (25^3 + 90k: 12.0 against 10.1), and its sums do not depend
+// on scheduling.  Without a MAS, whose own sums do, that holds up to 49,151 rows, so
+// that such a system's product and solves are the same bits in every run; it costs
+// up to 10% of an iteration (us, windows against the full BSR: 26^3 + 53k 20.4
+// against 19.4, 30^3 + 81k 22.7 (24.8), 36^3 + 140k 31.3 (35.9)).
+int spmv_auto_shape(int64_t B, bool use32, bool part_order)
 {
     if(env_shape_index() >= 0)
         return env_shape_index();
@@ -853,6 +856,8 @@ int spmv_auto_shape(int64_t B, bool use32)
     static constexpr Rule rules[] = {{196608, 0, 11}, {163841, 3, 3},  {114688, 15, 16}, {98304, 13, 14},
                                      {81921, 15, 14}, {57344, 13, 14}, {40960, 13, 12},  {16385, 12, 12}};
     const int64_t         rows    = B * 256 / std::max(1, device_cu_count());
+    if(!part_order && rows < 49152)
+        return spmv_shape_full;
     for(const Rule& r : rules)
         if(rows >= r.rows)
             return use32 ? r.f32 : (r.f64 == 0 ? default_shape_index() : r.f64);

@@ -302,7 +302,7 @@ def test_spmv_every_launch_shape(ctx, c1_contact, precision):
     ls.close()
 
 
-@pytest.mark.parametrize("B,rows", [(16384, (0, 0)), (57344, (64, 64)), (81920, (64, 64)), (81921, (128, 64)),
+@pytest.mark.parametrize("B,rows", [(16384, (0, 0)), (16385, (64, 64)), (49151, (64, 64)), (57344, (64, 64)), (81920, (64, 64)), (81921, (128, 64)),
                                     (98304, (64, 64)), (114687, (64, 64)), (114688, (128, 128)), (163840, (128, 128)),
                                     (163841, (256, 256)), (196607, (256, 256)), (196608, (512, 512))])
 def test_spmv_windows_by_size(ctx, B, rows):
@@ -310,6 +310,9 @@ def test_spmv_windows_by_size(ctx, B, rows):
     for precision, want in zip((abi.MI_FP64, abi.MI_FP32), rows):
         ls = LinearSystem(ctx, B, precision)
         i = np.arange(B, dtype=np.int32)
+        # a MAS over the first 16 rows puts the rows in a part order
+        ls.add_preconditioner(abi.MI_PRECOND_MAS, 0, 48, part_ids=np.zeros(16, np.int32),
+                              tets=np.array([[0, 1, 2, 3]], np.int32))
         ls.assemble(ctx.to_device(i), ctx.to_device(i), ctx.to_device(np.tile(np.eye(3).ravel(), (B, 1))))
         lay = ls.spmv_layout()
         assert lay["window_rows"] == want and lay["layout"] == ("window" if want else "full")
@@ -317,13 +320,17 @@ def test_spmv_windows_by_size(ctx, B, rows):
 
 
 @pytest.mark.parametrize("precision", [abi.MI_FP64, abi.MI_FP32])
-@pytest.mark.parametrize("grid,rows", [(25, 0), (26, 64), (39, 64)])
-def test_spmv_layout_by_size(ctx, precision, grid, rows):
+@pytest.mark.parametrize("grid,mas,rows", [(25, True, 0), (26, True, 64), (26, False, 0), (36, False, 0), (39, False, 64)])
+def test_spmv_layout_by_size(ctx, precision, grid, mas, rows):
     """the layout a system gets by its size (the full BSR up to 16,384 block
-    rows, 64-row windows above; the last window of 26^3 and 39^3 rows is a
-    partial one) and its product, against the oracle"""
+    rows, without a MAS 49,151, 64-row windows above; the last window of 26^3
+    and 39^3 rows is a partial one) and its product, against the oracle; the MAS
+    comes after the assembly and moves the rows to its layout"""
     s = synth.fem_system(grid, 2 * grid ** 2, seed=4)
     ls = assembled(ctx, s, precision)
+    if mas:
+        ls.add_preconditioner(abi.MI_PRECOND_MAS, 0, s.n, part_ids=s.part_ids, tets=s.tets)
+        ls.assemble_preconditioners()
     lay = ls.spmv_layout()
     assert lay["window_rows"] == rows and lay["layout"] == ("window" if rows else "full")
     orr, oc, ov, _ = O.convert_sym(s.block_rows, s.rows, s.cols, s.vals)
@@ -334,6 +341,35 @@ def test_spmv_layout_by_size(ctx, precision, grid, rows):
     tol = 1e-13 if precision == abi.MI_FP64 else 1e-6  # as test_spmv_dot
     assert np.abs(yd.numpy() - yref).max() <= tol * np.abs(yref).max()
     assert d == pytest.approx(dref, rel=tol * 10)
+    ls.close()
+
+
+@pytest.mark.parametrize("precision", [abi.MI_FP64, abi.MI_FP32])
+@pytest.mark.parametrize("shape,precond", [(abi.MI_SPMV_SHAPE_AUTO, "diag3"), (abi.MI_SPMV_SHAPE_FULL, "diag3"),
+                                           (abi.MI_SPMV_SHAPE_FULL, "mas")])
+def test_same_bits_in_every_run(ctx, shape, precond, precision):
+    """27^3 rows: the full BSR's products, by default without a MAS, are the same
+    bits whatever the scheduling, and so are the block Jacobi's solves"""
+    s = synth.fem_system(27, 40_000, seed=4)
+    ls = LinearSystem(ctx, s.block_rows, precision)
+    ls.set_spmv_shape(shape)
+    if precond == "mas":
+        ls.add_preconditioner(abi.MI_PRECOND_MAS, 0, s.n, part_ids=s.part_ids, tets=s.tets)
+    else:
+        ls.add_preconditioner(abi.MI_PRECOND_DIAG3, 0, s.n)
+    ls.assemble(ctx.to_device(s.rows), ctx.to_device(s.cols), ctx.to_device(s.vals))
+    ls.assemble_preconditioners()
+    b, v = ctx.to_device(s.rhs), ctx.to_device(np.random.default_rng(3).standard_normal(s.n))
+    y, x = ctx.alloc(s.n, np.float64), ctx.alloc(s.n, np.float64)
+    seen = set()
+    for _ in range(8):
+        ls.spmv(1.0, v, 0.0, y)
+        got = y.numpy().tobytes()
+        if precond == "diag3":
+            ls.solve(b, x, criterion=abi.MI_CRIT_REL_RESIDUAL, tol=1e-4)
+            got += x.numpy().tobytes()
+        seen.add(got)
+    assert len(seen) == 1
     ls.close()
 
 
