@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 def gpu_mas(ctx, s, precision=abi.MI_FP64, active_levels=0, invert=abi.MI_MAS_INVERT_SWEEP, shape=None):
-    """shape: the SpMV layout (None: by size, the full BSR below ~200k rows;
+    """shape: the SpMV layout (None: by size, the full BSR up to 16,384 rows;
     0: 512-row windows in the MAS part order, the PCG then iterating in it)"""
     ls = LinearSystem(ctx, s.block_rows)
     if shape is not None:
@@ -47,6 +47,36 @@ def test_mas_tables_and_clusters(ctx, grid, contacts, partition):
     # FP64 inverses (same sweep, FMA rounding)
     I = m.inverses()
     assert np.abs(g["inv"] - I).max() <= 1e-8 * np.abs(I).max()
+
+
+def one_cluster_per_range(m):
+    """per level from 1: do the vertices of every range of 256 partition slots have
+    their ancestors in one cluster (level 1: which no other range shares)?"""
+    t = m.tables()
+    part = t["real_to_part"]
+    in_part = part >= 0
+    ranges, out = part[in_part] // 256, []
+    for level in range(1, m.L):
+        pairs = np.unique(np.stack([ranges, t["coarse_tables"][in_part, level - 1] // 16]), axis=1)
+        one = np.unique(pairs[0]).size == pairs.shape[1]
+        out.append(bool(one and (level > 1 or np.unique(pairs[1]).size == pairs.shape[1])))
+    return out
+
+
+@pytest.mark.parametrize("grid,contacts,local", [(24, 3000, [True] * 4), (25, 3000, [True, False, True, True])])
+def test_mas_clusters_of_ranges(ctx, grid, contacts, local):
+    """the assembly by ranges of 256 slots, where every range pushes all levels in
+    LDS and where some have their ancestors in two clusters of level 2 (the push
+    launches then follow): the oracle's cluster matrices"""
+    s, (r, c, v) = system(grid, contacts, 11, "geometric")
+    ls, h = gpu_mas(ctx, s)
+    m = O.Mas(s.block_rows, s.part_ids, s.tets)
+    assert one_cluster_per_range(m) == local
+    m.assemble(r, c, v)
+    g, H = ls.mas_export(h), m.hessians()
+    # as test_mas_tables_and_clusters
+    assert np.allclose(g["hess"], H, rtol=1e-11, atol=1e-12 * np.abs(H).max())
+    ls.close()
 
 
 @pytest.mark.parametrize("precision,tol", [(abi.MI_FP64, 1e-9), (abi.MI_FP32, 2e-4)])

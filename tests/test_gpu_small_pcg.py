@@ -10,20 +10,23 @@ pytestmark = pytest.mark.gpu
 
 
 def solve_both(ctx, ls, b, tol=1e-8, **kw):
-    """one launch (the default), and use_graph = 0: plain launches"""
+    """one launch (the default; fits: does this system take it?), and use_graph = 0:
+    plain launches"""
     out = []
+    fits = kw.pop("fits", True)
     for use_graph in (1, 0):
         x = ctx.alloc(ls.n, np.float64)
         if "x_init" in kw:
             x.upload(kw["x0"])
         opts = {k: v for k, v in kw.items() if k != "x0"}
         st = ls.solve(b, x, tol=tol, use_graph=use_graph, true_residual=1, **opts)
+        assert (ls.one_launch() > 0) == (fits and use_graph == 1)
         out.append((st, x.numpy()))
     return out
 
 
-def check(ctx, ls, b, tol=1e-8, err=1e-6, **kw):
-    (s1, x1), (s0, x0) = solve_both(ctx, ls, b, tol, criterion=abi.MI_CRIT_REL_RESIDUAL, **kw)
+def check(ctx, ls, b, tol=1e-8, err=1e-6, criterion=abi.MI_CRIT_REL_RESIDUAL, **kw):
+    (s1, x1), (s0, x0) = solve_both(ctx, ls, b, tol, criterion=criterion, **kw)
     assert s1["converged"] == s0["converged"] == 1
     # rounding moves a stiff system's count: at most 10% more, the bound of
     # test_mas_pcg (with float inverses it takes up to 20% fewer: the launches
@@ -50,28 +53,31 @@ def dense_spd(B, per_row, seed):
     return rows, cols, np.concatenate([diag, v])
 
 
-@pytest.mark.parametrize("B,per_row", [(1, 1), (63, 4), (64, 4), (65, 4), (700, 20), (2500, 60), (5000, 130), (16384, 6)])
-def test_small_pcg_rows(ctx, B, per_row):
+@pytest.mark.parametrize("B,per_row,fits", [(1, 1, True), (63, 4, True), (64, 4, True), (65, 4, True), (700, 20, True),
+                                            (2500, 30, True), (8192, 20, True), (2500, 60, False), (5000, 130, False),
+                                            (16384, 6, True), (16385, 6, False)])
+def test_small_pcg_rows(ctx, B, per_row, fits):
     """one row, workgroups one row short of and past 64 rows, blocks past the
-    registers (3,072 per workgroup) and columns past LDS (2,048), and the most
-    rows it takes"""
+    registers (3,072 per workgroup; 3,900 here), columns past LDS (2,048; 2,300),
+    both, which it leaves to the launches, the most rows it takes and one more"""
     rows, cols, vals = dense_spd(B, per_row, seed=B)
     ls = LinearSystem(ctx, B)
     ls.assemble(ctx.to_device(rows), ctx.to_device(cols), ctx.to_device(vals))
     b = ctx.to_device(np.random.default_rng(1).standard_normal(3 * B))
     ls.add_preconditioner(abi.MI_PRECOND_DIAG3, 0, 3 * (B // 2))  # z = r on the other rows
     ls.assemble_preconditioners()
-    check(ctx, ls, b)
+    check(ctx, ls, b, fits=fits)
     ls.close()
 
 
 @pytest.mark.parametrize("precision,mas", [(abi.MI_FP64, abi.MI_FP64), (abi.MI_FP64, abi.MI_FP32),
                                            (abi.MI_FP32, abi.MI_FP32)])
 @pytest.mark.parametrize("grid,contacts,levels", [(2, 0, 0), (5, 40, 0), (9, 900, 0), (9, 900, 1), (9, 900, 2),
-                                                  (17, 2000, 0), (25, 0, 0)])
+                                                  (17, 2000, 0), (24, 0, 0), (25, 0, 0)])
 def test_small_pcg_mas(ctx, grid, contacts, levels, precision, mas):
-    """MAS over the whole vector at every kind of hierarchy (one cluster to six
-    levels), every level count, float and double storage"""
+    """MAS over the whole vector in hierarchies of two (2^3) to five levels (17^3,
+    24^3), with one and two of them applied, float and double storage; 24^3 has 13,824
+    partition slots, 25^3 18,928, past the 16,384 of one launch"""
     s = synth.fem_system(grid, contacts, seed=grid + 1)
     ls = LinearSystem(ctx, s.block_rows, precision)
     ls.assemble(ctx.to_device(s.rows), ctx.to_device(s.cols), ctx.to_device(s.vals))
@@ -80,15 +86,17 @@ def test_small_pcg_mas(ctx, grid, contacts, levels, precision, mas):
     ls.assemble_preconditioners()
     b = ctx.to_device(s.rhs)
     # contacts of four decades of stiffness: x to the residual times the condition
-    check(ctx, ls, b, err=1e-3)
-    # from a given x0, and the rz criterion
+    check(ctx, ls, b, err=1e-3, fits=grid < 25)
+    # from a given x0, and the rz criterion (r.z is about the residual's square)
     x0 = np.random.default_rng(3).standard_normal(s.n)
-    check(ctx, ls, b, err=1e-3, x_init=1, x0=x0)
+    check(ctx, ls, b, err=1e-3, x_init=1, x0=x0, fits=grid < 25)
+    check(ctx, ls, b, err=1e-3, tol=1e-16, criterion=abi.MI_CRIT_RZ_RATIO, fits=grid < 25)
     ls.close()
 
 
 def test_small_pcg_stops(ctx):
-    """the iteration cap, the interval counts and a NaN in b, as the launches"""
+    """the iteration cap, the interval counts, and a NaN in b, which is found before
+    the first iteration, as the launches"""
     s = synth.fem_system(9, 900, seed=2)
     ls = LinearSystem(ctx, s.block_rows)
     ls.assemble(ctx.to_device(s.rows), ctx.to_device(s.cols), ctx.to_device(s.vals))
@@ -220,13 +228,36 @@ def test_small_pcg_dense_rows(ctx, pre, hubs, reach, fits):
     ls.assemble_preconditioners()
     b = ctx.to_device(s.rhs)
     for _ in range(2):
-        check(ctx, ls, b)
-        x = ctx.alloc(s.n, np.float64)
-        ls.solve(b, x, criterion=abi.MI_CRIT_REL_RESIDUAL, tol=1e-8)
-        assert ls.one_launch() == (1 if fits else 0)
+        check(ctx, ls, b, fits=fits)
     free = [ctx.to_device(v) for v in (s.rows, s.cols, s.vals)]
     ls.assemble(*free)
     ls.assemble_preconditioners()
     ls.solve(b, ctx.alloc(s.n, np.float64), criterion=abi.MI_CRIT_REL_RESIDUAL, tol=1e-8)
     assert ls.one_launch() == 1
+    ls.close()
+
+
+@pytest.mark.parametrize("pre", ["diag3", "mas"])
+def test_small_pcg_not_finite(ctx, pre):
+    """a NaN in an off-diagonal block: r0.z0 is finite, the first iteration's r.z is
+    not, and the launch ends there with the launches' error"""
+    s = synth.fem_system(9, 900, seed=2)
+    vals = s.vals.copy()
+    # of two vertices in different parts: no preconditioner's cluster holds it
+    at = np.flatnonzero((s.rows != s.cols) & (s.part_ids[s.rows] != s.part_ids[s.cols]))[7]
+    vals[at, 4] = np.nan
+    ls = LinearSystem(ctx, s.block_rows)
+    ls.assemble(ctx.to_device(s.rows), ctx.to_device(s.cols), ctx.to_device(vals))
+    if pre == "mas":
+        ls.add_preconditioner(abi.MI_PRECOND_MAS, 0, s.n, part_ids=s.part_ids, tets=s.tets, active_levels=1)
+    else:
+        ls.add_preconditioner(abi.MI_PRECOND_DIAG3, 0, s.n)
+    ls.assemble_preconditioners()
+    b, text = ctx.to_device(s.rhs), []
+    for use_graph in (1, 0):
+        with pytest.raises(abi.MiError) as e:
+            ls.solve(b, ctx.alloc(s.n, np.float64), tol=1e-8, use_graph=use_graph)
+        assert e.value.code == abi.MI_ERR_NONFINITE and ls.one_launch() == use_graph
+        text.append(str(e.value))
+    assert "at iteration 1" in text[0] and "at iteration" in text[1]
     ls.close()
