@@ -15,10 +15,11 @@
 //     (the reference sums in atomic arrival order,
 //     fast_segmental_reduce.h:23-26);
 //   * values land in 9 SoA planes (see BsrMatrix);
-//   * one host read-back (the unique count, to size the outputs) instead of two;
-//   * the upper BCOO is then transposed (the same radix sort on col * B + row
-//     of the off-diagonal blocks) and merged row by row into a full BSR, so the
-//     SpMV is a pure row gather without atomics.
+//   * two host read-backs: the largest col - row, which chooses the sort key, and
+//     the unique count, which sizes the outputs;
+//   * the upper BCOO is then transposed (a stable radix sort of the off-diagonal
+//     blocks by column alone: they come in row order) and laid out for the SpMV,
+//     as a full BSR, a pure row gather without atomics, or in windows.
 #include "linsys.hpp"
 #include "segtile.hpp"
 

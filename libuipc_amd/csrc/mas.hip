@@ -22,7 +22,9 @@
 //            bank (FP64 atomics, wave-aggregated when few destinations repeat);
 //            the walk stops where the ancestors merge; where every level-1 bank is
 //            a 256-slot range, a workgroup per range sums its coarse clusters in
-//            LDS and does their pushes too;
+//            LDS and pushes level 0, and where besides every range's ancestors lie
+//            in one cluster per level above, all levels (grids of 16^3, 24^3, 33^3, 41^3 and
+//            64^3 in geometric parts; not 25^3, 43^3 or 50^3);
 //     push   level by level, the full sum of every group of nodes that share a
 //            parent becomes the parent's diagonal block (plain store; a parent's
 //            children all live in one bank).  This replaces the reference's

@@ -841,8 +841,9 @@ int spmv_default_shape()
 // against 9.1) or near (25^3 + 90k: 12.0 against 10.1), and its sums do not depend
 // on scheduling.  Without a MAS, whose own sums do, that holds up to 49,151 rows, so
 // that such a system's product and solves are the same bits in every run; it costs
-// up to 10% of an iteration (us, windows against the full BSR: 26^3 + 53k 20.4
-// against 19.4, 30^3 + 81k 22.7 (24.8), 36^3 + 140k 31.3 (35.9)).
+// up to 18% of an iteration (us, windows against the full BSR: 26^3 + 53k 20.4
+// against 19.4, 30^3 + 81k 22.7 (24.8), 36^3 + 140k 31.3 (35.9), 34^3 + 300k 37.3
+// (44.0), FP32 29.7 (29.1)).
 int spmv_auto_shape(int64_t B, bool use32, bool part_order)
 {
     if(env_shape_index() >= 0)
