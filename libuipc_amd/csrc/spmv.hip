@@ -833,13 +833,16 @@ int spmv_default_shape()
 // 128-row windows end where five workgroups per CU, all that fit, no longer hold
 // them in one round: whole PCG iterations at 54^3 + 1.2M (1,231 windows) FP64 113.7
 // (256-row windows 120.2), FP32 82.9 (92.3), at 55^3 + 1.3M (1,300) 126.9 (121.7) and 103.3
-// (93.5), 57^3 + 0.4M FP32 85.7 (79.4).  FP64 64-row windows end for the same reason at
-// 81,920 rows: 43^3 + 0.6M 72.4 (128 rows: 75.6), 44^3 + 0.65M 76.3 (75.3), until their
-// second round is well filled too, 48^3 + 0.84M 87.5 (88.7).
+// (93.5), 57^3 + 0.4M FP32 85.7 (79.4).  FP64 64-row windows meet the same line at
+// 81,920 rows, until their second round is well filled too (98,304).  Without a MAS they
+// give way there: 44^3 + 0.65M 68.5 (128 rows 65.0); in a part order the iteration is
+// the same (76.3, 75.3) and the product alone better, 44^3 + 0.19M 25.3 (26.6).
 // In the caller's order (no MAS) the same choices measured 35.9 (40.9) and 71.2
 // (78.5) in FP64.  Up to 16,384 rows the full BSR's row gather is as fast (20^3: 5.8
 // against 9.1) or near (25^3 + 90k: 12.0 against 10.1), and its sums do not depend
-// on scheduling.  Without a MAS, whose own sums do, that holds up to 49,151 rows, so
+// on scheduling.  Just above, a dense system's product alone is faster on it too (26^3 +
+// 134k 13.4 against 15.0, 28^3 + 167k 15.4 against 15.8), but an iteration in the part
+// order is not (27^3 + 150k 41.5 against 39.8).  Without a MAS, whose own sums do, that holds up to 49,151 rows, so
 // that such a system's product and solves are the same bits in every run; it costs
 // up to 18% of an iteration (us, windows against the full BSR: 26^3 + 53k 20.4
 // against 19.4, 30^3 + 81k 22.7 (24.8), 36^3 + 140k 31.3 (35.9), 34^3 + 300k 37.3
@@ -851,17 +854,21 @@ int spmv_auto_shape(int64_t B, bool use32, bool part_order)
     struct Rule
     {
         int64_t rows;  // from this many block rows on
-        int     f64, f32;
+        int     f64, f64_plain, f32;  // in a part order, in the caller's, either
     };
     // rows per CU (256 of them): 768, 640, 448, 384, 320, 224, 160, 64
-    static constexpr Rule rules[] = {{196608, 0, 11}, {163841, 3, 3},  {114688, 15, 16}, {98304, 13, 14},
-                                     {81921, 15, 14}, {57344, 13, 14}, {40960, 13, 12},  {16385, 12, 12}};
+    static constexpr Rule rules[] = {{196608, 0, 0, 11},   {163841, 3, 3, 3},   {114688, 15, 15, 16},
+                                     {98304, 13, 13, 14},  {81921, 13, 15, 14}, {57344, 13, 13, 14},
+                                     {40960, 13, 13, 12},  {16385, 12, 12, 12}};
     const int64_t         rows    = B * 256 / std::max(1, device_cu_count());
     if(!part_order && rows < 49152)
         return spmv_shape_full;
     for(const Rule& r : rules)
         if(rows >= r.rows)
-            return use32 ? r.f32 : (r.f64 == 0 ? default_shape_index() : r.f64);
+        {
+            const int k = use32 ? r.f32 : part_order ? r.f64 : r.f64_plain;
+            return k == 0 ? default_shape_index() : k;
+        }
     return spmv_shape_full;
 }
 

@@ -302,17 +302,21 @@ def test_spmv_every_launch_shape(ctx, c1_contact, precision):
     ls.close()
 
 
-@pytest.mark.parametrize("B,rows", [(16384, (0, 0)), (16385, (64, 64)), (49151, (64, 64)), (57344, (64, 64)), (81920, (64, 64)), (81921, (128, 64)),
-                                    (98304, (64, 64)), (114687, (64, 64)), (114688, (128, 128)), (163840, (128, 128)),
-                                    (163841, (256, 256)), (196607, (256, 256)), (196608, (512, 512))])
-def test_spmv_windows_by_size(ctx, B, rows):
+@pytest.mark.parametrize("B,mas,rows", [(16384, True, (0, 0)), (16385, True, (64, 64)), (49151, False, (0, 0)),
+                                        (49152, False, (64, 64)), (81920, False, (64, 64)), (81921, True, (64, 64)),
+                                        (81921, False, (128, 64)), (98303, False, (128, 64)), (98304, False, (64, 64)),
+                                        (114687, True, (64, 64)), (114688, True, (128, 128)),
+                                        (163840, True, (128, 128)), (163841, True, (256, 256)),
+                                        (196607, True, (256, 256)), (196608, True, (512, 512))])
+def test_spmv_windows_by_size(ctx, B, mas, rows):
     """the window sizes at the lines of the rule (FP64, FP32)"""
     for precision, want in zip((abi.MI_FP64, abi.MI_FP32), rows):
         ls = LinearSystem(ctx, B, precision)
         i = np.arange(B, dtype=np.int32)
         # a MAS over the first 16 rows puts the rows in a part order
-        ls.add_preconditioner(abi.MI_PRECOND_MAS, 0, 48, part_ids=np.zeros(16, np.int32),
-                              tets=np.array([[0, 1, 2, 3]], np.int32))
+        if mas:
+            ls.add_preconditioner(abi.MI_PRECOND_MAS, 0, 48, part_ids=np.zeros(16, np.int32),
+                                  tets=np.array([[0, 1, 2, 3]], np.int32))
         ls.assemble(ctx.to_device(i), ctx.to_device(i), ctx.to_device(np.tile(np.eye(3).ravel(), (B, 1))))
         lay = ls.spmv_layout()
         assert lay["window_rows"] == want and lay["layout"] == ("window" if want else "full")
