@@ -78,7 +78,9 @@ def tune_spmv_shape(ls: LinearSystem, x, reps: int = 20, shapes=None, margin: fl
     the reference fits its SpMV grid to each matrix (Spmv::fit_block_count,
     linear_system/spmv.cu:909-933).  The system's layout stays unless another
     is faster by more than `margin` (timing noise would otherwise flip
-    between near-equal layouts).  Returns {"best": k, "table": {k: {"us",
+    between near-equal layouts), or its last solve ran in one launch, which a
+    window layout rules out (16^3 rows with a MAS: 64-row windows give a product
+    in 5.9 us against 6.5, but a 20-iteration PCG solve in 500 us against 350).  Returns {"best": k, "table": {k: {"us",
     "threads", "rows", "per", "vec"}}}."""
     import numpy as np
 
@@ -90,6 +92,7 @@ def tune_spmv_shape(ls: LinearSystem, x, reps: int = 20, shapes=None, margin: fl
     info = spmv_shapes(ls.lib)["shapes"]
     lay0 = ls.spmv_layout()
     dflt = lay0["shape"] if lay0["layout"] == "window" else MI_SPMV_SHAPE_FULL  # the system's own layout
+    one_launch = ls.one_launch() > 0
     from .abi import MI_FP64
 
     if shapes is None:
@@ -120,7 +123,7 @@ def tune_spmv_shape(ls: LinearSystem, x, reps: int = 20, shapes=None, margin: fl
             product()
         table[k] = {"us": round(1e3 * ev.stop() / max(1, reps), 2), **desc}
     best = min(table, key=lambda k: table[k]["us"])
-    if dflt in table and table[best]["us"] > (1.0 - margin) * table[dflt]["us"]:
+    if dflt in table and (one_launch or table[best]["us"] > (1.0 - margin) * table[dflt]["us"]):
         best = dflt
     ls.set_spmv_shape(best, stream)
     ctx.synchronize()

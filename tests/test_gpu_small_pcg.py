@@ -261,3 +261,42 @@ def test_small_pcg_not_finite(ctx, pre):
         text.append(str(e.value))
     assert "at iteration 1" in text[0] and "at iteration" in text[1]
     ls.close()
+
+
+def test_small_pcg_survives_the_shape_tuner(ctx, monkeypatch):
+    """a system whose solves run in one launch keeps the full BSR when its SpMV
+    shapes are timed, also where the windows' products are faster (a timer that
+    makes every shape faster than the one before); one without a solve is free"""
+    from libuipc_amd import hip_events
+    from libuipc_amd.tune import tune_spmv_shape
+
+    class Timer:
+        shapes = 0
+
+        def __init__(self, stream):
+            pass
+
+        def start(self):
+            Timer.shapes += 1
+
+        def stop(self):
+            return 1.0 / Timer.shapes
+
+    monkeypatch.setattr(hip_events, "EventTimer", Timer)
+    s = synth.fem_system(16, 0, seed=2)
+    ls = LinearSystem(ctx, s.block_rows)
+    ls.add_preconditioner(abi.MI_PRECOND_MAS, 0, s.n, part_ids=s.part_ids, tets=s.tets)
+    ls.assemble(ctx.to_device(s.rows), ctx.to_device(s.cols), ctx.to_device(s.vals))
+    ls.assemble_preconditioners()
+    b, x = ctx.to_device(s.rhs), ctx.alloc(s.n, np.float64)
+    assert tune_spmv_shape(ls, b, reps=2)["best"] >= 0
+    ls.set_spmv_shape(abi.MI_SPMV_SHAPE_AUTO)
+    ls.assemble_preconditioners()
+    ls.solve(b, x, tol=1e-6)
+    assert ls.one_launch() == 1
+    Timer.shapes = 0
+    t = tune_spmv_shape(ls, b, reps=2)
+    assert t["best"] == abi.MI_SPMV_SHAPE_FULL and len(t["table"]) > 1
+    ls.solve(b, x, tol=1e-6)
+    assert ls.one_launch() == 1
+    ls.close()
